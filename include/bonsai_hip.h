@@ -378,7 +378,8 @@ int bh_pq2_embed_gather_rms(const uint8_t *table, size_t ne0, size_t n_rows,
  * magnitude (the summation order differs, as the reference's AVX2 path's
  * does).  Up to 4 tokens on rows of whole 1024-weight chunks (16-byte
  * aligned) the products keep x in LDS and use no scratch; otherwise they
- * use the library's per-device scratch (x fragments): such calls must not
+ * use the library's per-device scratch (x fragments; for large batches also
+ * up to 96 MB of unpacked weights, and partial sums): such calls must not
  * overlap on one device.
  * ------------------------------------------------------------------------- */
 

@@ -8,7 +8,10 @@
 // adds scale * block_sum to the row total; its AVX2 path reorders the same
 // sums (~1e-6 relative).  This file computes the same per-block structure
 // with MFMA tiles, in a different summation order (max relative difference
-// well below 1e-5 of the output's largest magnitude).
+// well below 1e-5 of the output's largest magnitude).  Up to 4 tokens, and
+// few outputs or many row tiles of up to 16 tokens, run here on the integer
+// matrix cores; other batches in pq2_mx.hip on the block-scaled ones; the f16
+// form below takes up to 4 tokens on rows that cannot be staged.
 //
 // Mapping onto v_mfma_f32_16x16x32_f16 (D = A * B + C, 16x16 output tile;
 // lane l holds A[l % 16][8 (l / 16) .. +7], B[8 (l / 16) .. +7][l % 16],
@@ -34,6 +37,7 @@
 #include <string>
 
 #include "common.hpp"
+#include "pq2_mx.hpp"
 
 namespace bh {
 namespace {
@@ -135,7 +139,7 @@ __global__ __launch_bounds__(kMmThreads) void pq2_mm_prep_kernel(PrepArgs a) {
 
 // ---------------------------------------------------------------------------
 // Main product.  Block = 4 waves; a wave owns NT 16-row weight tiles and the
-// block's MT token tiles.  Lane l: row n = l & 15 of each weight tile, lane
+// token tile (up to 16 tokens).  Lane l: row n = l & 15 of each weight tile, lane
 // group g = l >> 4 (code bytes 8g..8g+7 of every block).
 //
 // Weights are read two blocks (68 bytes, 17 dwords) at a time: with 4-byte
@@ -207,16 +211,15 @@ __device__ __forceinline__ BlockCodes block_codes(const PairData &d, int half) {
   return c;
 }
 
-template <int MT, int NT, bool ALDS>
+template <int NT, bool ALDS>
 __global__ __launch_bounds__(kMmThreads) void pq2_mm_kernel(MmArgs a) {
-  // ALDS (one token tile of at most kLdsTok tokens): the x side of the whole
+  // ALDS: the x side of the whole
   // product is staged in LDS once, fragments [kstep][piece][token][lane
   // group] followed by the block factors [block][lane group]
   extern __shared__ uint4 a_lds[];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int n = lane & 15, g = lane >> 4;
   const int row_wave = blockIdx.x * (4 * 16 * NT) + wave * 16 * NT;
-  const int tile0 = blockIdx.y * MT;
 
   const uint32_t *wp[NT];
 #pragma unroll
@@ -228,13 +231,13 @@ __global__ __launch_bounds__(kMmThreads) void pq2_mm_kernel(MmArgs a) {
   // Row m of an MFMA result depends on row m of A only, so the lanes of a
   // tile's absent tokens may feed any fragment (their rows are never
   // stored): they read a real token's (ALDS) or unwritten scratch.
-  const uint4 *af = a.afrag + static_cast<size_t>(tile0) * a.n_ksteps * 2 * 64 + lane;
-  const float4 *binv_g = a.binv + (static_cast<size_t>(tile0) * a.nblk * 4 + g) * 2;
+  const uint4 *af = a.afrag + lane;
+  const float4 *binv_g = a.binv + g * 2;
   const uint4 *al = a_lds;
   const float4 *binv_l = nullptr;
   int lds_tok_stride = 0;
   if constexpr (ALDS) {
-    const int nt = a.n_tok;  // <= kLdsTok: tile 0 only
+    const int nt = a.n_tok;
     const int total = a.n_ksteps * 2 * nt * 4;
     for (int i = threadIdx.x; i < total; i += kMmThreads) {
       const int gq = i & 3, rest = i >> 2;
@@ -249,74 +252,59 @@ __global__ __launch_bounds__(kMmThreads) void pq2_mm_kernel(MmArgs a) {
   }
   if constexpr (ALDS) __syncthreads();  // x staging visible to every wave
 
-  f4v tot[MT][NT];
+  f4v tot[NT];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int t = 0; t < NT; ++t) tot[mt][t] = f4v{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < NT; ++t) tot[t] = f4v{0.f, 0.f, 0.f, 0.f};
 
   auto do_block = [&](const BlockCodes(&bc)[NT], int b) {
-    f4v acc[MT][NT], acc_lo[MT][NT];  // hi and lo pieces: two independent MFMA chains
+    f4v acc[NT], acc_lo[NT];  // hi and lo pieces: two independent MFMA chains
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int t = 0; t < NT; ++t) acc[mt][t] = acc_lo[mt][t] = f4v{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < NT; ++t) acc[t] = acc_lo[t] = f4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int ks = 4 * b + i;
-      h8 ahi[MT], alo[MT];
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        if constexpr (ALDS) {
-          const uint4 *pl = al + (2 * ks) * lds_tok_stride;
-          ahi[mt] = __builtin_bit_cast(h8, pl[0]);
-          alo[mt] = __builtin_bit_cast(h8, pl[lds_tok_stride]);
-        } else {
-          const uint4 *pg = af + (static_cast<size_t>(mt) * a.n_ksteps + ks) * 2 * 64;
-          ahi[mt] = __builtin_bit_cast(h8, pg[0]);
-          alo[mt] = __builtin_bit_cast(h8, pg[64]);
-        }
+      h8 ahi, alo;
+      if constexpr (ALDS) {
+        const uint4 *pl = al + (2 * ks) * lds_tok_stride;
+        ahi = __builtin_bit_cast(h8, pl[0]);
+        alo = __builtin_bit_cast(h8, pl[lds_tok_stride]);
+      } else {
+        const uint4 *pg = af + static_cast<size_t>(ks) * 2 * 64;
+        ahi = __builtin_bit_cast(h8, pg[0]);
+        alo = __builtin_bit_cast(h8, pg[64]);
       }
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         const uint32_t d = bc[t].cd[i >> 1];
         const h8 bf = decode_fp4(d, i);
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          acc[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi[mt], bf, acc[mt][t], 0, 0, 0);
-          acc_lo[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo[mt], bf, acc_lo[mt][t], 0, 0, 0);
-        }
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bf, acc[t], 0, 0, 0);
+        acc_lo[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bf, acc_lo[t], 0, 0, 0);
       }
     }
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) acc[mt][t][q] = acc[mt][t][q] + acc_lo[mt][t][q];
+      for (int q = 0; q < 4; ++q) acc[t][q] = acc[t][q] + acc_lo[t][q];
     // src/kernels.rs:651: acc += scale * block_acc -- block_acc arrives
     // multiplied by the block's 2^e, so the factor is scale * 2^-e (exact)
+    float4 bi, bs;
+    if constexpr (ALDS) {
+      bi = binv_l[b * 8];
+      bs = binv_l[b * 8 + 1];
+    } else {
+      bi = binv_g[static_cast<size_t>(b) * 8];
+      bs = binv_g[static_cast<size_t>(b) * 8 + 1];
+    }
+    const float inv[4] = {bi.x, bi.y, bi.z, bi.w};
+    const float xs[4] = {bs.x, bs.y, bs.z, bs.w};
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      float4 bi, bs;
-      if constexpr (ALDS) {
-        bi = binv_l[b * 8];
-        bs = binv_l[b * 8 + 1];
-      } else {
-        bi = binv_g[(static_cast<size_t>(mt) * a.nblk + b) * 8];
-        bs = binv_g[(static_cast<size_t>(mt) * a.nblk + b) * 8 + 1];
-      }
-      const float inv[4] = {bi.x, bi.y, bi.z, bi.w};
-      const float xs[4] = {bs.x, bs.y, bs.z, bs.w};
+    for (int t = 0; t < NT; ++t) {
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const float f = bc[t].sc * inv[q];
-          const float blk = acc[mt][t][q] - xs[q];
-          const float prod = f * blk;
-          tot[mt][t][q] = tot[mt][t][q] + prod;
-        }
+      for (int q = 0; q < 4; ++q) {
+        const float f = bc[t].sc * inv[q];
+        const float blk = acc[t][q] - xs[q];
+        const float prod = f * blk;
+        tot[t][q] = tot[t][q] + prod;
       }
     }
   };
@@ -348,29 +336,24 @@ __global__ __launch_bounds__(kMmThreads) void pq2_mm_kernel(MmArgs a) {
     if (p + 1 < npairs) run_pair(pb, p + 1);
   }
 
-  // lane holds tokens 4g..4g+3 of each token tile, row n of each weight tile
+  // lane holds tokens 4g..4g+3, row n of each weight tile
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
+  for (int q = 0; q < 4; ++q) {
+    const int m = 4 * g + q;
+    if (m >= a.n_tok) continue;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int m = 16 * (tile0 + mt) + 4 * g + q;
-      if (m >= a.n_tok) continue;
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const int row = row_wave + 16 * t + n;
-        if (row < a.n_rows) a.y[static_cast<size_t>(m) * a.y_stride + row] = tot[mt][t][q];
-      }
+    for (int t = 0; t < NT; ++t) {
+      const int row = row_wave + 16 * t + n;
+      if (row < a.n_rows) a.y[static_cast<size_t>(m) * a.y_stride + row] = tot[t][q];
     }
   }
 }
 
 // ---------------------------------------------------------------------------
-// Staged product (16-byte aligned rows, block count a multiple of 8): each
-// wave streams its 16 rows through LDS in chunks of 8 blocks (272 bytes per
-// row, 17 dwordx4 loads per row, so consecutive lanes read consecutive 16
-// bytes of a row), then every lane reads its fragment codes from LDS.  One
-// chunk is in flight in registers while the previous one is consumed; the
-// stage is private to the wave (in-order LDS, no block barrier).
+// Staged weights (16-byte aligned rows, block count a multiple of 8): a wave
+// streams its 16 rows through LDS in chunks of 8 blocks (272 bytes per row,
+// 17 dwordx4 loads per row, so consecutive lanes read consecutive 16 bytes of
+// a row), then every lane reads its fragment codes from LDS.
 // ---------------------------------------------------------------------------
 constexpr int kStageBlocks = 8;
 constexpr int kStageRowBytes = kPq2Blk * kStageBlocks;          // 272
@@ -381,150 +364,6 @@ constexpr size_t kStageWaveBytes = 16 * kStageStride;           // 4480
 
 __device__ __forceinline__ uint32_t lds_u32(const uint8_t *p) {
   return *reinterpret_cast<const uint32_t *>(p);
-}
-
-// TOKQ: accumulator elements per lane that can hold a real token (the tile
-// has at most 4 * TOKQ ... lanes of groups g >= 1 hold tokens >= 4, so with
-// n_tok <= TOKQ only elements q < TOKQ of group 0 carry results).
-template <bool ALDS, int TOKQ>
-__global__ __launch_bounds__(kMmThreads) void pq2_mm_staged_kernel(MmArgs a) {
-  extern __shared__ uint4 smem[];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int n = lane & 15, g = lane >> 4;
-  const int row_wave = blockIdx.x * 64 + wave * 16;
-
-  // x side: whole product in LDS (ALDS) or fragments from global
-  const uint4 *af = a.afrag + lane;
-  const uint4 *al = smem;
-  const float4 *binv_l = nullptr;
-  int lds_tok_stride = 0;
-  size_t a_words = 0;  // uint4 slots used by the ALDS area
-  if constexpr (ALDS) {
-    const int nt = a.n_tok;
-    const int total = a.n_ksteps * 2 * nt * 4;
-    for (int i = threadIdx.x; i < total; i += kMmThreads) {
-      const int gq = i & 3, rest = i >> 2;
-      const int m = rest % nt, kp = rest / nt;
-      smem[i] = a.afrag[static_cast<size_t>(kp) * 64 + 16 * gq + m];
-    }
-    float4 *bl = reinterpret_cast<float4 *>(smem + total);
-    for (int i = threadIdx.x; i < a.nblk * 8; i += kMmThreads) bl[i] = a.binv[i];
-    al = smem + (n < nt ? n : 0) * 4 + g;
-    lds_tok_stride = nt * 4;
-    binv_l = bl + 2 * g;
-    a_words = static_cast<size_t>(total) + static_cast<size_t>(a.nblk) * 8;
-  }
-  uint8_t *stage = reinterpret_cast<uint8_t *>(smem + a_words) + wave * kStageWaveBytes;
-
-  // this lane's share of a chunk: float4 slot k covers row r_k, piece c_k
-  const uint8_t *src[kStageLoads];
-  int dst[kStageLoads];
-  bool live[kStageLoads];
-#pragma unroll
-  for (int k = 0; k < kStageLoads; ++k) {
-    const int idx = lane + 64 * k;
-    live[k] = idx < 16 * kStageF4;
-    const int r = live[k] ? idx / kStageF4 : 0, c16 = live[k] ? idx % kStageF4 : 0;
-    int row = row_wave + r;
-    row = row < a.n_rows ? row : a.n_rows - 1;  // tail rows read a valid row, store nothing
-    src[k] = a.w + static_cast<size_t>(row) * a.row_bytes + 16 * c16;
-    dst[k] = r * kStageStride + 16 * c16;
-  }
-  uint4 regs[kStageLoads];
-  auto gload = [&](int chunk) {
-#pragma unroll
-    for (int k = 0; k < kStageLoads; ++k)
-      if (live[k]) regs[k] = *reinterpret_cast<const uint4 *>(src[k] + static_cast<size_t>(chunk) * kStageRowBytes);
-  };
-  auto lstore = [&]() {
-#pragma unroll
-    for (int k = 0; k < kStageLoads; ++k) {
-      if (live[k]) {
-        uint2 *d = reinterpret_cast<uint2 *>(stage + dst[k]);  // 8-byte aligned
-        d[0] = make_uint2(regs[k].x, regs[k].y);
-        d[1] = make_uint2(regs[k].z, regs[k].w);
-      }
-    }
-  };
-  f4v tot = f4v{0.f, 0.f, 0.f, 0.f};
-
-  const int n_chunks = a.nblk / kStageBlocks;
-  gload(0);
-  if constexpr (ALDS) __syncthreads();  // x staging visible to every wave
-  lstore();
-  if (n_chunks > 1) gload(1);
-  for (int c = 0; c < n_chunks; ++c) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const uint8_t *rowp = stage + n * kStageStride;
-    for (int bb = 0; bb < kStageBlocks; ++bb) {
-      const int b = c * kStageBlocks + bb;
-      const uint8_t *blk = rowp + kPq2Blk * bb;
-      BlockCodes bc;
-      if ((bb & 1) == 0) {  // block starts on a dword: codes are 2 bytes in
-        const uint32_t e0 = lds_u32(blk + 8 * g), e1 = lds_u32(blk + 8 * g + 4),
-                       e2 = lds_u32(blk + 8 * g + 8);
-        bc.cd[0] = __builtin_amdgcn_alignbyte(e1, e0, 2);
-        bc.cd[1] = __builtin_amdgcn_alignbyte(e2, e1, 2);
-        bc.sc = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(lds_u32(blk))));
-      } else {  // block starts 2 bytes into a dword: codes are dword-aligned
-        bc.cd[0] = lds_u32(blk + 2 + 8 * g);
-        bc.cd[1] = lds_u32(blk + 6 + 8 * g);
-        bc.sc = static_cast<float>(
-            __builtin_bit_cast(_Float16, static_cast<uint16_t>(lds_u32(blk - 2) >> 16)));
-      }
-      f4v acc = f4v{0.f, 0.f, 0.f, 0.f}, acc_lo = acc;  // two independent MFMA chains
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int ks = 4 * b + i;
-        h8 ahi, alo;
-        if constexpr (ALDS) {
-          const uint4 *pl = al + (2 * ks) * lds_tok_stride;
-          ahi = __builtin_bit_cast(h8, pl[0]);
-          alo = __builtin_bit_cast(h8, pl[lds_tok_stride]);
-        } else {
-          const uint4 *pg = af + static_cast<size_t>(ks) * 2 * 64;
-          ahi = __builtin_bit_cast(h8, pg[0]);
-          alo = __builtin_bit_cast(h8, pg[64]);
-        }
-        const uint32_t d = bc.cd[i >> 1];
-        const h8 bf = decode_fp4(d, i);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bf, acc, 0, 0, 0);
-        acc_lo = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bf, acc_lo, 0, 0, 0);
-      }
-#pragma unroll
-      for (int q = 0; q < TOKQ; ++q) acc[q] = acc[q] + acc_lo[q];
-      float4 bi, bs;
-      if constexpr (ALDS) {
-        bi = binv_l[b * 8];
-        bs = binv_l[b * 8 + 1];
-      } else {
-        bi = a.binv[(static_cast<size_t>(b) * 4 + g) * 2];
-        bs = a.binv[(static_cast<size_t>(b) * 4 + g) * 2 + 1];
-      }
-      const float inv[4] = {bi.x, bi.y, bi.z, bi.w};
-      const float xs[4] = {bs.x, bs.y, bs.z, bs.w};
-#pragma unroll
-      for (int q = 0; q < TOKQ; ++q) {
-        const float f = bc.sc * inv[q];  // src/kernels.rs:651, block scale * 2^-e
-        const float blk = acc[q] - xs[q];
-        const float prod = f * blk;
-        tot[q] = tot[q] + prod;
-      }
-    }
-    if (c + 1 < n_chunks) {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      lstore();  // chunk c + 1 replaces chunk c (this wave finished reading it)
-      if (c + 2 < n_chunks) gload(c + 2);
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < TOKQ; ++q) {
-    const int m = 4 * g + q;
-    const int row = row_wave + n;
-    if (m < a.n_tok && row < a.n_rows) a.y[static_cast<size_t>(m) * a.y_stride + row] = tot[q];
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1334,40 +1173,22 @@ __global__ void fill_zero_kernel(float *y, size_t n) {
   if (i < n) y[i] = 0.0f;
 }
 
-constexpr int kLdsTok = 4;                 // token counts staged whole in LDS
-constexpr size_t kLdsABytes = 104 * 1024;  // their LDS budget (with 4 wave stages: 121 KB)
+constexpr size_t kLdsABytes = 104 * 1024;  // LDS budget of a whole x side (with 4 wave stages: 121 KB)
 
-template <int MT, int NT, bool ALDS = false>
-int launch_mm(const MmArgs &a, int n_tiles, hipStream_t st) {
+template <int NT, bool ALDS = false>
+int launch_mm(const MmArgs &a, hipStream_t st) {
   const unsigned gx = static_cast<unsigned>((a.n_rows + 64 * NT - 1) / (64 * NT));
-  const unsigned gy = static_cast<unsigned>((n_tiles + MT - 1) / MT);
   size_t lds = 0;
   if constexpr (ALDS) {
     lds = static_cast<size_t>(a.n_ksteps) * 2 * a.n_tok * 4 * sizeof(uint4) +
           static_cast<size_t>(a.nblk) * 8 * sizeof(float4);
-    if (int e = check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(pq2_mm_kernel<MT, NT, true>),
+    if (int e = check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(pq2_mm_kernel<NT, true>),
                                               hipFuncAttributeMaxDynamicSharedMemorySize,
                                               static_cast<int>(kLdsABytes)),
                           "hipFuncSetAttribute"))
       return e;
   }
-  BH_LAUNCH((pq2_mm_kernel<MT, NT, ALDS>), dim3(gx, gy), kMmThreads, lds, st, a);
-  return ok();
-}
-
-template <bool ALDS, int TOKQ>
-int launch_staged(const MmArgs &a, hipStream_t st) {
-  const unsigned gx = static_cast<unsigned>((a.n_rows + 63) / 64);
-  size_t lds = 4 * kStageWaveBytes;
-  if constexpr (ALDS)
-    lds += static_cast<size_t>(a.n_ksteps) * 2 * a.n_tok * 4 * sizeof(uint4) +
-           static_cast<size_t>(a.nblk) * 8 * sizeof(float4);
-  if (int e = check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(pq2_mm_staged_kernel<ALDS, TOKQ>),
-                                            hipFuncAttributeMaxDynamicSharedMemorySize,
-                                            static_cast<int>(kLdsABytes + 4 * kStageWaveBytes)),
-                        "hipFuncSetAttribute"))
-    return e;
-  BH_LAUNCH((pq2_mm_staged_kernel<ALDS, TOKQ>), gx, kMmThreads, lds, st, a);
+  BH_LAUNCH((pq2_mm_kernel<NT, ALDS>), gx, kMmThreads, lds, st, a);
   return ok();
 }
 
@@ -1532,15 +1353,27 @@ int pq2_mm(const uint8_t *w, size_t ne0, size_t n_rows, const float *x, size_t n
                            (nblk * kI8Tok * sizeof(float2) + 15) / 16 * 16;
     if (a_bytes <= kLdsABytes) return pq2_i8<false>(w, ne0, n_rows, x, n_tok, y, a_bytes, st);
   }
-  if (stageable && n_tok > static_cast<size_t>(kI8Tok)) return pq2_gemm_i8(w, ne0, n_rows, x, n_tok, y, st);
+  // more tokens, and rows so long that their digits don't fit LDS
+  // ([5120 x 17408], 4 tokens: 51 -> 27 us): the block-scaled matrix cores --
+  // except where the integer form is still faster: one pass over a matrix of
+  // many row tiles ([248320 x 5120], 16 tokens: 138 us against 146; [17408 x
+  // 5120]: 30 against 25), and short rows with few outputs, where its fewer
+  // launches count (2048 columns, 3000 x 300 outputs: 22 us against 25; 8000 x
+  // 300: 39 against 33).
+  if (n_tok > static_cast<size_t>(kI8Tok) || stageable) {
+    // items of the forms below and above, which index them in int
+    if (n_tok * nblk * (stageable ? 8 : 16) > static_cast<size_t>(INT32_MAX) - kMmThreads)
+      return fail(BH_ERR_SHAPE, "pq2_matmul_n: n_tok * ne0 too large for one call");
+    const bool i8 = (n_tok <= 16 && n_rows >= 32768) || (nblk <= 16 && n_rows * n_tok <= (1u << 20));
+    if (stageable && n_tok > static_cast<size_t>(kI8Tok) && i8)
+      return pq2_gemm_i8(w, ne0, n_rows, x, n_tok, y, st);
+    return pq2_mx_gemm(w, ne0, n_rows, x, n_tok, y, st);
+  }
+  // f16 hi / lo: up to 4 tokens on rows that cannot be staged
   const int n_ksteps = static_cast<int>(ne0 / 32);
-  const int n_tiles = static_cast<int>((n_tok + 15) / 16);
-  const int mt = n_tiles >= 4 ? 4 : (n_tiles >= 2 ? 2 : 1);
-  const int tiles_padded = (n_tiles + mt - 1) / mt * mt;
-  // scratch: A fragments, then the per-(token, block) powers of two
-  const size_t frag_bytes = static_cast<size_t>(tiles_padded) * n_ksteps * 2 * 64 * sizeof(uint4);
+  const size_t frag_bytes = static_cast<size_t>(n_ksteps) * 2 * 64 * sizeof(uint4);
   const size_t binv_off = (frag_bytes + 255) / 256 * 256;
-  const size_t binv_bytes = static_cast<size_t>(tiles_padded) * nblk * 8 * sizeof(float4);
+  const size_t binv_bytes = nblk * 8 * sizeof(float4);
   char *scratch = static_cast<char *>(device_scratch(binv_off + binv_bytes, kScratchMatmul, st));
   if (scratch == nullptr) return BH_ERR_HIP;
   PrepArgs pa{x, reinterpret_cast<uint4 *>(scratch), reinterpret_cast<float *>(scratch + binv_off),
@@ -1556,21 +1389,11 @@ int pq2_mm(const uint8_t *w, size_t ne0, size_t n_rows, const float *x, size_t n
            static_cast<int>(n_rows)};
   // a wave takes 4 row tiles when that still leaves >= 2 blocks per CU
   const bool wide = n_rows >= static_cast<size_t>(256) * 2 * 256;
-  const bool staged = nblk % kStageBlocks == 0 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0 &&
-                      row_bytes % 16 == 0 && n_tiles == 1;
-  const bool a_in_lds = n_tok <= kLdsTok && static_cast<size_t>(n_ksteps) * 2 * n_tok * 4 * sizeof(uint4) +
-                                                 nblk * 8 * sizeof(float4) <= kLdsABytes;
-  if (staged) {
-    if (a_in_lds) return n_tok == 1 ? launch_staged<true, 1>(a, st) : launch_staged<true, 4>(a, st);
-    return launch_staged<false, 4>(a, st);
-  }
+  const bool a_in_lds = static_cast<size_t>(n_ksteps) * 2 * n_tok * 4 * sizeof(uint4) +
+                            nblk * 8 * sizeof(float4) <= kLdsABytes;
   if (a_in_lds)
-    return wide ? launch_mm<1, 4, true>(a, n_tiles, st) : launch_mm<1, 1, true>(a, n_tiles, st);
-  switch (mt) {
-    case 4: return wide ? launch_mm<4, 4>(a, n_tiles, st) : launch_mm<4, 1>(a, n_tiles, st);
-    case 2: return wide ? launch_mm<2, 4>(a, n_tiles, st) : launch_mm<2, 1>(a, n_tiles, st);
-    default: return wide ? launch_mm<1, 4>(a, n_tiles, st) : launch_mm<1, 1>(a, n_tiles, st);
-  }
+    return wide ? launch_mm<4, true>(a, st) : launch_mm<1, true>(a, st);
+  return wide ? launch_mm<4>(a, st) : launch_mm<1>(a, st);
 }
 
 // Byte length of rows [0, base_row + n_rows), or false on overflow.

@@ -283,3 +283,65 @@ def test_host_mirrors(bh, oracle, synth):
     bh.check(lib.bh_host_pq2_matmul_n(table.ctypes.data, table.size, ne0, 0, n_rows,
                                       x.ctypes.data, x.size, 3, ym.ctypes.data, ym.size))
     assert _per_token_err(ym, oracle.pq2_matmul_n(table, ne0, n_rows, x)) <= TOL
+
+
+@pytest.mark.parametrize("ne0,n_rows,n_tok", [
+    (256, 40, 5),         # one pair of blocks, less than a row tile of 32 and its wave
+    (768, 300, 33),       # 6 blocks (rows not 16-byte aligned), a second token tile of one
+    (2304, 8200, 31),     # 18 blocks, a ragged last panel
+    (5120, 17408, 17),    # blocks in parts: raw, one row tile a wave
+    (5120, 4100, 96),     # ragged panel, three token tiles
+    (5120, 17408, 64),    # raw, two row tiles a wave
+    (5120, 70000, 20),    # raw, several rounds of workgroups
+    (5120, 1500, 3000),   # unpacked tiles, fewer than the CUs
+    (5120, 8200, 1100),   # unpacked: a whole round, the rest in parts, ragged both ways
+    (5120, 40000, 450),   # unpacked in two passes over the rows
+    (17408, 512, 2), (17408, 700, 4),  # digits too long for LDS
+])
+def test_matmul_block_scaled(bh, synth, dev, ne0, n_rows, n_tok):
+    """The block-scaled forms at the edges of their tiles against 64-bit sums
+    of the same weights.  x has 24-bit digits and every f32 sum rounds once,
+    so the 2-norm error stays within sqrt(10) roundings of a block's sum and
+    sqrt(blocks) of a row's: (sqrt(10) + sqrt(nblk)) 2^-24."""
+    import torch
+    _say("block-scaled", ne0, n_rows, n_tok)
+    g = torch.Generator(device=dev)
+    g.manual_seed(ne0 + n_rows + n_tok)
+    nblk = ne0 // 128
+    codes = torch.randint(0, 4, (n_rows, nblk, 32, 4), device=dev, generator=g, dtype=torch.uint8)
+    d = (torch.randn((n_rows, nblk), device=dev, generator=g) * 0.02).to(torch.float16)
+    tab = torch.empty((n_rows, nblk, 34), device=dev, dtype=torch.uint8)
+    tab[..., :2] = d.view(torch.uint8).view(n_rows, nblk, 2)
+    tab[..., 2:] = (codes[..., 0] | (codes[..., 1] << 2) | (codes[..., 2] << 4) | (codes[..., 3] << 6))
+    x = torch.randn((n_tok, ne0), device=dev, generator=g)
+    y = torch.full((n_tok, n_rows), float("nan"), device=dev)
+    bh.pq2_matmul_n(tab.view(-1), ne0, n_rows, x, out=y)
+    err = ref2 = 0.0
+    for r in range(0, n_rows, 8192):
+        w = (codes[r:r + 8192].double() - 1).view(-1, nblk, 128) * d[r:r + 8192].double()[..., None]
+        ref = x.double() @ w.view(-1, ne0).T
+        err += float((y[:, r:r + 8192].double() - ref).square().sum())
+        ref2 += float(ref.square().sum())
+    rel = (err / ref2) ** 0.5
+    _say("  rel", rel)
+    assert rel <= (10 ** 0.5 + nblk ** 0.5) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("n_tok", [20, 1100])
+def test_matmul_zero_weight_hides_outlier(bh, synth, dev, n_tok):
+    """A weight of zero takes nothing from its x, however large: a token with
+    one value 1e20 times the rest, met by code 1 in every row, gives what it
+    gives with that value zero, bit for bit (on both block-scaled forms)."""
+    import torch
+    ne0, n_rows = 5120, 2000
+    tab = torch.from_numpy(synth.pq2_table(synth.Rng(31), n_rows, ne0)).to(dev)
+    col = 1234  # byte 2 + (1234 % 128) / 4 of block 9, code 2: bits 4-5
+    byte = 34 * (col // 128) + 2 + (col % 128) // 4
+    tab[:, byte] = (tab[:, byte] & ~(3 << 4 * 1)) | (1 << 4) if col % 4 == 2 else tab[:, byte]
+    x = torch.from_numpy(synth.Rng(32).normal(n_tok * ne0).reshape(n_tok, ne0)).to(dev)
+    # the column's group of 32 keeps its scale: only the outlier stands in it
+    x[:, col // 32 * 32:col // 32 * 32 + 32] = 0
+    base = _h(bh.pq2_matmul_n(tab.view(-1), ne0, n_rows, x))
+    x[:, col] = 1e20
+    got = _h(bh.pq2_matmul_n(tab.view(-1), ne0, n_rows, x))
+    assert np.array_equal(got, base)
