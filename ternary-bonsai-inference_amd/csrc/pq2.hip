@@ -20,25 +20,19 @@
 // Fused RMSNorm, bit-exact.  The reference sums the 5120 squares of a row
 // one after another in f32 (src/kernels.rs:65-68); on quantised embedding
 // rows that sequence drifts ~1e-5 from any tree-ordered sum, so the fused
-// kernel reproduces the sequence itself.  A block owns kFusedRows rows: its
-// rows are staged in LDS, "producer" waves decode them chunk by chunk (256
-// or 512 columns), store the embedding rows and write the f32 squares to an LDS
-// ring laid out column-major, while one "chain" wave adds them in column
-// order, one row per lane -- the same additions in the same order as the
-// CPU, so the norm output is bit-identical too.  The chain (5120 dependent
-// adds, ~21 us) runs under the embedding stores; the norm rows are then
-// decoded a second time from LDS and stored.  Batches of at least 16 rows per
-// CU take two launches instead, with flat writers: the row scales come from
-// runs of identical squares evaluated in closed form (seqsum.hpp), computed
-// by the first blocks of the launch that writes the embedding rows, and a
-// second launch writes the norm rows.
-//
-// Bit-exactness: the f16 scale is widened with integer arithmetic (exact for
-// all patterns, see half_bits_to_f32_bits) and the weight is one multiply of
-// an exact small integer by it, so the product is exactly the CPU's.
+// kernels reproduce the sequence itself.  On ternary codes a 128-block adds
+// d*d as many times as it has codes other than 1, a run that seqsum.hpp
+// evaluates exactly without its additions.  Up to 16 rows per CU one launch:
+// a workgroup per row, one wave taking the row's runs by turns (a lane per
+// block) under the embedding stores, then the norm row.  Its time is the
+// launch, the row's first touch and about 15 turns: T = 1 8.4 us, 256 11.5,
+// 2048 17.2 (5.0 TB/s of 86.7 MB); a chain of the 5120 additions, a lane per
+// row, took 22.7, 27.8 and 29.5.  Longer batches: two launches of flat
+// writers (below), the sums walked a lane per row under the stores.
 #include <hip/hip_runtime.h>
 
 #include <string>
+#include <type_traits>
 
 #include "common.hpp"
 #include "seqsum.hpp"
@@ -50,21 +44,6 @@ constexpr int kBlock = 256;
 constexpr int kPq2Block = 34;
 constexpr size_t kMaxSeqSmem = 128 * 1024;  // LDS cap of a fused block (gfx950: 160 KB per CU)
 
-
-// ---------------------------------------------------------------------------
-// Fused gather + RMSNorm with the reference's sequential f32 sum of squares:
-// one launch, one block of kFusedThreads lanes per kFusedRows output rows.
-// ---------------------------------------------------------------------------
-// Block shapes: kFusedRows rows per block (= chain lanes), kFusedThreads
-// lanes (wave 0 the chain, the others producers) and kChunkQ float4 columns
-// per chunk of the ring (one barrier per chunk).
-
-// LDS of a block of `rows` rows: staged packed rows, the f32 scale of every
-// (row, 128-block) and the two-chunk ring of squared weights.
-size_t fused_smem_bytes(size_t row_bytes, int rows, int chunk_q) {
-  const size_t n_scales = (rows * (row_bytes / kPq2Block) + 3) & ~static_cast<size_t>(3);
-  return rows * row_bytes + n_scales * sizeof(float) + 2 * chunk_q * (rows + 1) * sizeof(float4);
-}
 
 struct GatherArgs {
   const uint8_t *table;
@@ -78,134 +57,6 @@ struct GatherArgs {
   float eps;
 };
 
-// Phase 1 (column chunks of 4 kChunkQ weights, ring of squares):
-//   producer waves decode chunk c of all the block's rows, store those
-//   embedding float4 and write their f32 squares to the ring, column-major;
-//   the chain wave (lane = row) adds chunk c-1 in column order -- the same
-//   additions in the same order as src/kernels.rs:65-68, so the row scale
-//   is bit-identical to the CPU's.  The chain is latency-bound (~10 cycles
-//   per dependent add, ~21 us for 5120 weights) and runs under the stores.
-// Phase 2: all waves decode the rows again from LDS and store the norm rows
-//   (v * scale) * w (src/kernels.rs:71-73), flat over the block's rows.
-template <int kFusedRows, int kFusedThreads, int kChunkQ>
-__global__ __launch_bounds__(kFusedThreads) void pq2_gather_rms_kernel(GatherArgs a) {
-  constexpr int kRingStride = kFusedRows + 1;  // float4 slots per column (padded)
-  extern __shared__ uint4 smem[];
-  __shared__ int row_ok[kFusedRows];
-  __shared__ float row_scale[kFusedRows];
-  const int rb16 = a.row_bytes >> 4;
-  const int nblk = a.row_bytes / kPq2Block;
-  uint4 *stage = smem;                                                  // [rows][rb16]
-  float *scales = reinterpret_cast<float *>(smem + kFusedRows * rb16);  // [rows][nblk]
-  float4 *ring = reinterpret_cast<float4 *>(scales + ((kFusedRows * nblk + 3) & ~3));
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6;
-  const int lane = tid & 63;
-  const size_t row0 = static_cast<size_t>(blockIdx.x) * kFusedRows;
-  const int nr = (a.n_ids - static_cast<int>(row0)) < kFusedRows ? a.n_ids - static_cast<int>(row0)
-                                                                 : kFusedRows;
-  const int n4 = a.ne0 >> 2;
-
-  if (tid < kFusedRows) {
-    int okr = 0;
-    if (tid < nr) {
-      const uint32_t id = a.ids[row0 + tid];
-      okr = id < a.n_rows;
-      if (!okr && a.bad_id != nullptr) *a.bad_id = id;
-    }
-    row_ok[tid] = okr;
-  }
-  for (int i = tid; i < nr * rb16; i += kFusedThreads) {
-    const int r = i / rb16;
-    const uint32_t id = a.ids[row0 + r];
-    if (id < a.n_rows)
-      stage[i] = reinterpret_cast<const uint4 *>(a.table + static_cast<size_t>(id) * a.row_bytes)[i - r * rb16];
-  }
-  __syncthreads();
-  // f32 scale of every staged 128-block (the f16 bits kept in the scale slot
-  // would be needed only for non-finite scales, which are re-read from the row)
-  for (int i = tid; i < nr * nblk; i += kFusedThreads) {
-    const int r = i / nblk;
-    const uint8_t *bp = reinterpret_cast<const uint8_t *>(stage + r * rb16) + (i - r * nblk) * kPq2Block;
-    const uint32_t h = static_cast<uint32_t>(bp[0]) | (static_cast<uint32_t>(bp[1]) << 8);
-    scales[i] = __uint_as_float(half_bits_to_f32_bits(h));
-  }
-  __syncthreads();
-
-  const int n_chunks = (n4 + kChunkQ - 1) / kChunkQ;
-  float ss = 0.0f;  // chain lane `lane` accumulates row `lane`
-  for (int c = 0; c <= n_chunks; ++c) {
-    if (wave != 0) {
-      if (c < n_chunks) {
-        float4 *dst = ring + (c & 1) * (kChunkQ * kRingStride);
-        for (int i = tid - 64; i < kFusedRows * kChunkQ; i += kFusedThreads - 64) {
-          const int r = i / kChunkQ;  // lanes walk a row's kChunkQ columns: long store runs
-          const int q = i - r * kChunkQ;
-          const int f = c * kChunkQ + q;
-          float4 t = make_float4(0.f, 0.f, 0.f, 0.f);  // adding +0 leaves a sum unchanged
-          if (r < nr && f < n4) {
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (row_ok[r]) {
-              const uint8_t *rowb = reinterpret_cast<const uint8_t *>(stage + r * rb16);
-              const int b = f >> 5;
-              const uint32_t h = static_cast<uint32_t>(rowb[b * kPq2Block]) |
-                                 (static_cast<uint32_t>(rowb[b * kPq2Block + 1]) << 8);
-              const uint32_t code = rowb[b * kPq2Block + 2 + (f & 31)];
-              const float sc = scales[r * nblk + b];
-              const bool finite = (h & 0x7c00u) != 0x7c00u;
-              v = make_float4(pq2_weight(code & 3u, sc, finite), pq2_weight((code >> 2) & 3u, sc, finite),
-                              pq2_weight((code >> 4) & 3u, sc, finite), pq2_weight((code >> 6) & 3u, sc, finite));
-              t = make_float4(v.x * v.x, v.y * v.y, v.z * v.z, v.w * v.w);
-            }
-            store_stream(reinterpret_cast<float4 *>(a.out) + (row0 + r) * n4 + f, v);
-          }
-          dst[q * kRingStride + r] = t;
-        }
-      }
-    } else if (c > 0 && lane < kFusedRows) {
-      const float4 *src = ring + ((c - 1) & 1) * (kChunkQ * kRingStride);
-#pragma unroll 8
-      for (int q = 0; q < kChunkQ; ++q) {
-        const float4 t = src[q * kRingStride + lane];
-        ss += t.x;
-        ss += t.y;
-        ss += t.z;
-        ss += t.w;
-      }
-    }
-    __syncthreads();
-  }
-  if (wave == 0 && lane < kFusedRows) {
-    // src/kernels.rs:69-70: mean = ss / n; scale = 1 / sqrt(mean + eps)
-    row_scale[lane] = 1.0f / sqrtf(ss / static_cast<float>(a.ne0) + a.eps);
-  }
-  __syncthreads();
-
-  const float4 *w4 = reinterpret_cast<const float4 *>(a.w);
-  float4 *on = reinterpret_cast<float4 *>(a.out_norm) + row0 * n4;
-  const int total = nr * n4;
-  for (int i = tid; i < total; i += kFusedThreads) {
-    const int r = i / n4;
-    const int f = i - r * n4;
-    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (row_ok[r]) {
-      const uint8_t *rowb = reinterpret_cast<const uint8_t *>(stage + r * rb16);
-      const int b = f >> 5;
-      const uint32_t h = static_cast<uint32_t>(rowb[b * kPq2Block]) |
-                         (static_cast<uint32_t>(rowb[b * kPq2Block + 1]) << 8);
-      const uint32_t code = rowb[b * kPq2Block + 2 + (f & 31)];
-      const float sc = scales[r * nblk + b];
-      const bool finite = (h & 0x7c00u) != 0x7c00u;
-      const float4 v = make_float4(pq2_weight(code & 3u, sc, finite), pq2_weight((code >> 2) & 3u, sc, finite),
-                                   pq2_weight((code >> 4) & 3u, sc, finite), pq2_weight((code >> 6) & 3u, sc, finite));
-      const float4 wv = w4[f];
-      const float rs = row_scale[r];
-      o = make_float4((v.x * rs) * wv.x, (v.y * rs) * wv.y, (v.z * rs) * wv.z, (v.w * rs) * wv.w);
-    }
-    store_stream(on + i, o);
-  }
-}
-
 // Decodes float4 f of the packed row at `rowb` straight from global memory
 // (the scale halfword and one code byte; the row is 16-byte aligned and a
 // block starts on an even byte, so the halfword load is aligned).
@@ -218,6 +69,142 @@ __device__ __forceinline__ float4 decode4_global(const uint8_t *rowb, int f) {
   return make_float4(pq2_weight(c & 3u, scale, finite), pq2_weight((c >> 2) & 3u, scale, finite),
                      pq2_weight((c >> 4) & 3u, scale, finite),
                      pq2_weight((c >> 6) & 3u, scale, finite));
+}
+
+// ---------------------------------------------------------------------------
+// Gather + RMSNorm, one workgroup per row: wave 0 forms the row's sum of
+// squares -- one lane per 128-block (windows of 64 blocks), by turns -- while
+// the other waves write the embedding row; then all write the norm row.
+// ---------------------------------------------------------------------------
+constexpr int kRowThreads = 256;
+
+// Inclusive prefix sum over the wave's 64 lanes (all active): DPP row shifts,
+// then the last lane of each 16-lane row and of the lower half passed on.
+__device__ __forceinline__ uint32_t wave_prefix(uint32_t v) {
+  auto add = [&](auto ctrl, auto rows) {
+    v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), decltype(ctrl)::value,
+                                                           decltype(rows)::value, 0xF, false));
+  };
+  add(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xF>{});  // row_shr:1
+  add(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xF>{});
+  add(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xF>{});
+  add(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xF>{});
+  add(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xA>{});  // row_bcast:15
+  add(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xC>{});  // row_bcast:31
+  return v;
+}
+
+// The reference's sequential f32 sum of squares of the packed row, bit for
+// bit, on one whole wave.
+__device__ __forceinline__ float wave_row_ss(const uint8_t *row, int ne0, int nblk) {
+  const int lane = threadIdx.x & 63;
+  float s = 0.0f;
+  for (int b0 = 0; b0 < nblk; b0 += 64) {
+    const int b = b0 + lane;
+    float x = 0.0f;
+    uint32_t n = 0, by_hand = 0;
+    if (b < nblk) {
+      // the block's 34 bytes as eight aligned words and a halfword
+      const bool even = (b & 1) == 0;
+      const uint8_t *blk = row + static_cast<size_t>(b) * kPq2Block;
+      const uint32_t *w32 = reinterpret_cast<const uint32_t *>(blk + (even ? 0 : 2));
+      const uint32_t h16 = *reinterpret_cast<const uint16_t *>(blk + (even ? 32 : 0));
+      uint32_t dw[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) dw[k] = w32[k];
+      const uint32_t h = even ? (dw[0] & 0xffffu) : h16;
+      const int valid = ne0 - b * 128 < 128 ? ne0 - b * 128 : 128;
+      uint32_t ones = 0, threes = 0;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {  // 16 codes a word
+        const uint32_t nx = k < 7 ? dw[k < 7 ? k + 1 : 0] : h16;
+        const uint32_t w = even ? ((dw[k] >> 16) | (nx << 16)) : dw[k];
+        const int lo = valid - 16 * k;
+        const uint32_t mask =
+            lo >= 16 ? 0x55555555u : (lo <= 0 ? 0u : 0x55555555u & ((1u << (2 * lo)) - 1u));
+        const uint32_t t = w ^ 0x55555555u;  // code 1 -> 00
+        ones += __popc(~(t | (t >> 1)) & mask);
+        threes |= w & (w >> 1) & mask;
+      }
+      const float d = __uint_as_float(half_bits_to_f32_bits(h));
+      x = d * d;
+      n = x != 0.0f ? static_cast<uint32_t>(valid) - ones : 0u;  // d = 0: squares of +0
+      // a square of 4 d d, or a non-finite scale: weight by weight
+      by_hand = threes != 0u || (h & 0x7c00u) == 0x7c00u;
+      if (by_hand) n = 1;
+    }
+    for (;;) {
+      const uint32_t sb = __builtin_amdgcn_readfirstlane(__float_as_uint(s));
+      const SeqUnits u = seq_units(static_cast<int>(sb >> 23), x);
+      const uint32_t inc = n != 0u && by_hand == 0u ? seq_units_added(n, u) : 0u;
+      const uint32_t upto = wave_prefix(inc);
+      const uint32_t start = sb + (upto - inc);
+      const SeqStep step = seq_step(start, x, n, u);
+      const uint64_t stay = __ballot(n != 0u && (by_hand != 0u || !step.whole));
+      if (stay == 0u) {
+        s = __uint_as_float(sb + __builtin_amdgcn_readlane(upto, 63));
+        break;
+      }
+      const int f = __builtin_ctzll(stay);
+      uint32_t left = 0;
+      if (__builtin_amdgcn_readlane(by_hand, f) != 0) {
+        // src/kernels.rs:65-68: lane j squares weights j and j + 64
+        s = __uint_as_float(__builtin_amdgcn_readlane(start, f));
+        const uint8_t *blk = row + static_cast<size_t>(b0 + f) * kPq2Block;
+        const uint32_t h = *reinterpret_cast<const uint16_t *>(blk);
+        const float sc = __uint_as_float(half_bits_to_f32_bits(h));
+        const bool finite = (h & 0x7c00u) != 0x7c00u;
+        const int valid = ne0 - (b0 + f) * 128 < 128 ? ne0 - (b0 + f) * 128 : 128;
+        const float v0 = pq2_weight((blk[2 + (lane >> 2)] >> ((lane & 3) * 2)) & 3u, sc, finite);
+        const float v1 = pq2_weight((blk[18 + (lane >> 2)] >> ((lane & 3) * 2)) & 3u, sc, finite);
+        const uint32_t q0 = __float_as_uint(v0 * v0), q1 = __float_as_uint(v1 * v1);
+        for (int j = 0; j < valid; ++j)
+          s += __uint_as_float(j < 64 ? __builtin_amdgcn_readlane(q0, j)
+                                      : __builtin_amdgcn_readlane(q1, j - 64));
+      } else {
+        s = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(step.s), f));
+        left = __builtin_amdgcn_readlane(step.left, f);
+      }
+      n = lane < f ? 0u : (lane == f ? left : n);
+    }
+  }
+  return s;
+}
+
+__global__ __launch_bounds__(kRowThreads) void pq2_gather_row_kernel(GatherArgs a) {
+  __shared__ float row_scale;
+  const size_t t = blockIdx.x;
+  const uint32_t id = a.ids[t];
+  const int n4 = a.ne0 >> 2;
+  float4 *oe = reinterpret_cast<float4 *>(a.out) + t * n4;
+  float4 *on = reinterpret_cast<float4 *>(a.out_norm) + t * n4;
+  if (id >= a.n_rows) {
+    if (threadIdx.x == 0 && a.bad_id != nullptr) *a.bad_id = id;
+    for (int f = threadIdx.x; f < n4; f += kRowThreads) {
+      store_stream(oe + f, make_float4(0.f, 0.f, 0.f, 0.f));
+      store_stream(on + f, make_float4(0.f, 0.f, 0.f, 0.f));
+    }
+    return;
+  }
+  const uint8_t *row = a.table + static_cast<size_t>(id) * a.row_bytes;
+  if (threadIdx.x < 64) {
+    __builtin_amdgcn_s_setprio(3);  // the other waves wait for this one
+    const float ss = wave_row_ss(row, a.ne0, a.row_bytes / kPq2Block);
+    // src/kernels.rs:69-70: mean = ss / n; scale = 1 / sqrt(mean + eps)
+    if (threadIdx.x == 0) row_scale = 1.0f / sqrtf(ss / static_cast<float>(a.ne0) + a.eps);
+    __builtin_amdgcn_s_setprio(0);
+  } else {
+    for (int f = threadIdx.x - 64; f < n4; f += kRowThreads - 64) store_stream(oe + f, decode4_global(row, f));
+  }
+  __syncthreads();
+  const float rs = row_scale;
+  for (int f = threadIdx.x; f < n4; f += kRowThreads) {
+    const float4 wv = reinterpret_cast<const float4 *>(a.w)[f];
+    const float4 v = decode4_global(row, f);
+    // src/kernels.rs:71-73
+    store_stream(on + f, make_float4((v.x * rs) * wv.x, (v.y * rs) * wv.y, (v.z * rs) * wv.z,
+                                     (v.w * rs) * wv.w));
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -526,11 +513,10 @@ int gather_impl(const uint8_t *table, size_t ne0, size_t n_rows, const uint32_t 
   const size_t cus = device_cu_count();
   if (rows_ok && norm && row_bytes % 16 == 0 && n_ids >= 16 * cus &&
       scale_smem_bytes(row_bytes) <= kMaxSeqSmem) {
-    // Long batches: row scales + embedding rows, then the norm rows (two
-    // flat writers).  The scale walk (~20 us of dependent steps) hides under
-    // the embedding stores only when there are enough of them: measured at
-    // T=8192 55.5-64 us against 69-72 for the one-launch kernel below, at
-    // T=2048 32.0 against 30.0 (so shorter batches stay on that kernel).
+    // Long batches: row scales + embedding rows, then the norm rows (two flat
+    // writers, which stream faster than a workgroup's two rows one after the
+    // other).  Measured against the kernel below (us): T = 4096 36 / 34, 6000
+    // 43 / 49, 8192 56 / 66.
     float *scales = static_cast<float *>(device_scratch(n_ids * sizeof(float), kScratchGather, st));
     if (scales == nullptr) return BH_ERR_HIP;
     const size_t smem = scale_smem_bytes(row_bytes);
@@ -547,30 +533,8 @@ int gather_impl(const uint8_t *table, size_t ne0, size_t n_rows, const uint32_t 
     BH_LAUNCH(pq2_norm_write_kernel, 8 * e_per, 256, 0, st, ga, scales, e_per);
     return ok();
   }
-  if (rows_ok && norm && row_bytes % 16 == 0 && fused_smem_bytes(row_bytes, 16, 128) <= kMaxSeqSmem) {
-    // 16 rows per block while that still gives every CU a block; fewer rows
-    // per block (more blocks) for short batches: the chain's latency is the
-    // same for any number of rows, the rest of a block's work is not.
-    // Measured (us, T=2048 / 8192, chunks of 32 float4): 16 rows x 1024
-    // lanes 39.0 / 70.3, 8 x 1024 34.6 / 81, 8 x 512 37.0 / 70.7, 4 x 512
-    // 35.1 / 85, 4 x 256 38.6 / 69.  Longer chunks (fewer barriers on the
-    // chain's path): 8 rows, chunks of 64 / 128 float4 33.3 / 32.7 at
-    // T=2048; 16 rows, 64: 70.2 at T=8192 (128: 80.5).
-    const int rows = n_ids >= 16 * cus ? 16 : (n_ids >= 8 * cus ? 8 : 4);
-    auto launch = [&](auto kern, int r, int threads, int chunk_q) -> int {
-      const size_t smem = fused_smem_bytes(row_bytes, r, chunk_q);
-      if (int e = check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                                hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                static_cast<int>(smem)),
-                            "hipFuncSetAttribute"))
-        return e;
-      const unsigned fgrid = static_cast<unsigned>((n_ids + r - 1) / r);
-      BH_LAUNCH(kern, fgrid, threads, smem, st, ga);
-      return ok();
-    };
-    if (rows == 16) return launch(pq2_gather_rms_kernel<16, 1024, 64>, 16, 1024, 64);
-    if (rows == 8) return launch(pq2_gather_rms_kernel<8, 1024, 128>, 8, 1024, 128);
-    return launch(pq2_gather_rms_kernel<4, 512, 128>, 4, 512, 128);
+  if (rows_ok && norm && row_bytes % 4 == 0) {  // a block's codes are whole aligned words
+    BH_LAUNCH(pq2_gather_row_kernel, grid, kRowThreads, 0, st, ga);
   } else {
     if (norm) {
       BH_LAUNCH((pq2_gather_loop_kernel<true>), grid, kBlock, 0, st, table, row_bytes,
