@@ -28,6 +28,8 @@
 // scaling, one block per (position chunk, 128-row tile, kv head)); over an
 // f32 cache read by 8 or more row tiles per kv head the cache is first
 // split into f16 hi / lo once (attn_kv_split_kernel) instead of per block.
+// Blocks of many position tiles over an f16 or a pre-split cache take the
+// 32-row form (mq_wide_body).
 //
 // Generic path (any hd and grouping, any alignment): one block per (query,
 // head) computes the scores, the reference's softmax (f32 max, expf, f64
@@ -954,8 +956,9 @@ struct MqArgs {
   // f32 cache pre-split by attn_kv_split_kernel (PRE): K as f16 hi / lo
   // halves in the cache's layout with its per-position factors 2^-b; V per
   // (32-position tile, kv head) as [dim][32 halves in vcol order], hi then
-  // lo, with the tile's shift; unused otherwise
-  const uint16_t *kh, *kl, *vh;
+  // lo, with the tile's shift; or, by attn_kv_record_kernel, a record of the
+  // staged operand arrays with the factors of its positions; unused otherwise
+  const uint16_t *kh, *kl, *vh, *rec;
   const float *ks;
   const int *vsh;
 };
@@ -990,6 +993,34 @@ __device__ __forceinline__ void split_hl(float x, _Float16 &h, _Float16 &l) {
 // fragment is one 16-byte LDS read.
 __device__ __forceinline__ int vcol(int p) { return p < 16 ? 8 * (p >> 2) + (p & 3) : 8 * ((p - 16) >> 2) + 4 + (p & 3); }
 
+// The (chunk, row tile, kv head) of a multi-query block.  XCD-aware
+// numbering: workgroups go to the 8 XCDs round robin by id, so the row tiles
+// of one (chunk, kv head) get ids 8 apart -- the same XCD, dispatched
+// together -- and share the K/V tiles in that XCD's L2.
+__device__ __forceinline__ void mq_block(const MqArgs &a, int tiles_r, int &c, int &t, int &g) {
+  const int b = blockIdx.x;
+  const int n_groups = a.n_chunks * a.n_kv;  // (chunk, kv head) pairs
+  const int full = n_groups / 8 * 8;         // groups placed 8 at a time
+  const int x = b % 8, jb = b / 8;
+  int q;
+  if (a.n_chunks == 1) {
+    // one chunk (every position in one block, e.g. a causal prefill): the
+    // row tiles longest-first, kv heads interleaved, so the tiles that see
+    // the most positions start in the first round instead of the last
+    t = tiles_r - 1 - b / a.n_kv;
+    q = b % a.n_kv;
+  } else if (jb < (full / 8) * tiles_r) {
+    q = (jb / tiles_r) * 8 + x;
+    t = jb % tiles_r;
+  } else {  // the last n_groups % 8 groups, in plain order
+    const int rest = b - full * tiles_r;
+    q = full + rest / tiles_r;
+    t = rest % tiles_r;
+  }
+  c = q % a.n_chunks;
+  g = q / a.n_chunks;
+}
+
 // PB > 0: a planar-quantized cache of PB-bit indices (src/kvquant.rs).  The
 // tile's K and V values are the centroids of the packed indices, looked up
 // while staging (V's times its row norm, or V's f32 rows when VQ is false),
@@ -1010,35 +1041,10 @@ __device__ __forceinline__ void mq_body(const MqArgs &a, const float *cent, cons
   __shared__ float sKs[kMqTile];  // 2^-b of each staged K row
   __shared__ unsigned sVmax[2];   // bits of a tile's largest |v| (non-negative floats order as ints), by tile parity
   __shared__ float sC[PL ? 256 : 1];  // the centroids
-  // XCD-aware numbering: workgroups go to the 8 XCDs round robin by id, so
-  // the row tiles of one (chunk, kv head) get ids 8 apart -- the same XCD,
-  // dispatched together -- and share the K/V tiles in that XCD's L2.
   const int R = a.n_q * a.rep;
   const int tiles_r = (R + kMqRows - 1) / kMqRows;
   int c, t, g;
-  {
-    const int b = blockIdx.x;
-    const int n_groups = a.n_chunks * a.n_kv;  // (chunk, kv head) pairs
-    const int full = n_groups / 8 * 8;         // groups placed 8 at a time
-    const int x = b % 8, jb = b / 8;
-    int q;
-    if (a.n_chunks == 1) {
-      // one chunk (every position in one block, e.g. a causal prefill): the
-      // row tiles longest-first, kv heads interleaved, so the tiles that see
-      // the most positions start in the first round instead of the last
-      t = tiles_r - 1 - b / a.n_kv;
-      q = b % a.n_kv;
-    } else if (jb < (full / 8) * tiles_r) {
-      q = (jb / tiles_r) * 8 + x;
-      t = jb % tiles_r;
-    } else {  // the last n_groups % 8 groups, in plain order
-      const int rest = b - full * tiles_r;
-      q = full + rest / tiles_r;
-      t = rest % tiles_r;
-    }
-    c = q % a.n_chunks;
-    g = q / a.n_chunks;
-  }
+  mq_block(a, tiles_r, c, t, g);
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, r16 = l & 15, grp = l >> 4;
   const int rho = t * kMqRows + w * 16 + r16;
   const bool valid = rho < R;
@@ -1551,6 +1557,520 @@ __global__ __launch_bounds__(256) void attn_kv_split_kernel(const float *kc, con
   }
 }
 
+// ---- 32-row form of the multi-query kernel ----------------------------------
+//
+// The same blocks, products and softmax as mq_body with four waves of 32 rows
+// on v_mfma_f32_32x32x16_f16.  mq_body is bound by LDS reads and by its two
+// barriers a tile: eight waves of 16 rows read every staged K and V byte
+// eight times, for matrix instructions that run at half the rate of the
+// 32-row ones.  Here a staged byte is read four times, q's 128 registers and
+// the 128 accumulators live in the accumulation registers (one wave per SIMD,
+// 512 registers), both buffers of a tile take one barrier, and the loop is
+// pipelined by a tile: K of the next tile is multiplied beside this tile's
+// exponentials, V of this tile beside the next tile's masks and the stores of
+// the tiles in flight.  What bounds it now is instruction issue: a tile's
+// 64 products (f16) take 2048 cycles and its ~450 other vector instructions
+// about as many, of which half hides.
+// Measured, 24 / 4 heads: f16 cache, 333 queries at 4000: 102 us (16-row form
+// 122), at 12000: 245 (start of the tile loop to its end 2.3 us a tile
+// against 2.9); f32, 2048 queries from position 0: 230 us (270).  Relative
+// error against 64-bit arithmetic there 3.0e-7 (3.9e-7: the small cross
+// products have their own accumulator).
+constexpr int kWideThreads = 256;             // 4 waves, one per SIMD
+constexpr size_t kWideMinTiles = 8;           // position tiles per block from which this form is taken
+constexpr int kWideArr = 32 * kHd;            // halves of one operand array of a tile (16 KB)
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// Lane-order address (in halves) of a tile's operand pieces of eight halves.
+// K: position p, dims 8 c .. 8 c + 7 (k-step c / 2, lane half c % 2); V: dim
+// d, piece pp = 2 ks + half of the position order vpos below.  A piece sits
+// at its MFMA lane's place, with its place within eight lanes exchanged by an
+// XOR so that the staging stores of eight lanes fall in eight bank groups.
+__device__ __forceinline__ int wide_k(int p, int c) {
+  return ((c >> 1) * 64 + (c & 1) * 32 + (p ^ (c & 7))) * 8;
+}
+__device__ __forceinline__ int wide_v(int d, int pp) {
+  const int m = d & 31;
+  return (((d >> 5) * 2 + (pp >> 1)) * 64 + (pp & 1) * 32 + (m ^ ((m >> 3) & 3))) * 8;
+}
+// position of half j (0..7) of V piece pp: the order in which a lane half
+// holds the positions of its S^T fragment
+__device__ __forceinline__ int wide_vpos(int pp, int j) {
+  return 16 * (pp >> 1) + 8 * (j >> 2) + 4 * (pp & 1) + (j & 3);
+}
+__device__ __forceinline__ float pair_max(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float pair_sum(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+template <bool PRE>
+__device__ __forceinline__ void mq_wide_body(const MqArgs &a) {
+  constexpr int kParts = PRE ? 2 : 1;  // hi, lo
+  // staged K and V tiles, two buffers each: sT[K or V][buffer][hi, lo]
+  __shared__ __attribute__((aligned(16))) _Float16 sT[2][2][kParts * kWideArr];
+  __shared__ __attribute__((aligned(16))) float sKs[2][PRE ? kMqTile : 4];
+  const int R = a.n_q * a.rep;
+  const int tiles_r = (R + kMqRows - 1) / kMqRows;
+  int c, t, g;
+  mq_block(a, tiles_r, c, t, g);
+  // (divisions run on the vector unit; descriptors and bases want scalars)
+  c = __builtin_amdgcn_readfirstlane(c);
+  t = __builtin_amdgcn_readfirstlane(t);
+  g = __builtin_amdgcn_readfirstlane(g);
+  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, r32 = l & 31, h = l >> 5;
+  const int rho = t * kMqRows + w * 32 + r32;
+  const bool valid = rho < R;
+  const int qi = valid ? rho / a.rep : 0;
+  const int head = g * a.rep + (valid ? rho % a.rep : 0);
+  const size_t limit = valid ? a.pos0 + qi + 1 : 0;  // this row sees positions < limit
+  const int last_row = (t + 1) * kMqRows - 1 < R - 1 ? (t + 1) * kMqRows - 1 : R - 1;
+  const size_t lim_blk = a.pos0 + __builtin_amdgcn_readfirstlane(last_row / a.rep) + 1;
+  const size_t beg = static_cast<size_t>(c) * a.chunk;
+  const size_t end = beg + a.chunk < lim_blk ? beg + a.chunk : lim_blk;
+  const size_t part = (static_cast<size_t>(qi) * a.n_head + head) * a.n_chunks + c;
+  if (beg >= end) {  // no position of this chunk is visible to the tile
+    if (valid && a.out != nullptr) {
+      // (not reached: a one-chunk tile sees position 0) the merge's 0 / 0
+      f32x4 *dst = reinterpret_cast<f32x4 *>(a.out + (static_cast<size_t>(qi) * a.n_head + head) * kHd);
+      const float nan = __builtin_nanf("");
+#pragma unroll
+      for (int k = 0; k < 32; ++k) dst[2 * k + h] = f32x4{nan, nan, nan, nan};
+    } else if (valid) {
+      if (h == 0) {
+        a.pm[part] = -INFINITY;
+        a.pl[part] = 0.0f;
+      }
+      f32x4 *acc = reinterpret_cast<f32x4 *>(a.pacc + part * kHd);
+#pragma unroll
+      for (int k = 0; k < 32; ++k) acc[2 * k + h] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    return;
+  }
+  // q row fragments: dims 16 s + 8 h .. +7 of row rho, scaled and split
+  // (they pass through LDS: fragments that are read from LDS stay in the
+  // accumulation registers, which VALU results do not)
+  half8 qh[16], ql[16];
+  int qa = 0;
+  {
+    half8 *qs = reinterpret_cast<half8 *>(&sT[0][0][0]) + tid;
+    const f32x4 *qr = reinterpret_cast<const f32x4 *>(
+        a.q + (static_cast<size_t>(qi) * a.n_head + head) * kHd + 8 * h);
+    f32x4 v[32];
+#pragma unroll
+    for (int s = 0; s < 16; ++s) {
+      v[2 * s] = valid ? qr[4 * s] : f32x4{0.f, 0.f, 0.f, 0.f};
+      v[2 * s + 1] = valid ? qr[4 * s + 1] : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    float m = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 32; ++k)
+      m = fmaxf(m, fmaxf(fmaxf(fabsf(v[k].x), fabsf(v[k].y)), fmaxf(fabsf(v[k].z), fabsf(v[k].w))));
+    qa = split_shift(pair_max(m));
+    const float f = ldexpf(1.0f, qa);
+#pragma unroll
+    for (int part_hl = 0; part_hl < 2; ++part_hl) {
+#pragma unroll
+      for (int s = 0; s < 16; ++s) {
+        half8 x;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          _Float16 hi, lo;
+          split_hl(v[2 * s + (k >> 2)][k & 3] * f, hi, lo);
+          x[k] = part_hl == 0 ? hi : lo;
+        }
+        qs[kWideThreads * s] = x;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int s = 0; s < 16; ++s) (part_hl == 0 ? qh : ql)[s] = qs[kWideThreads * s];
+      __syncthreads();
+    }
+  }
+  const float qunscale = ldexpf(a.scale, -qa);  // scores: S' * 2^-a * 2^-b * (1/sqrtf(hd))
+
+  f32x16 o[8];
+#pragma unroll
+  for (int dt = 0; dt < 8; ++dt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[dt][i] = 0.0f;
+  float run_m = -INFINITY, run_l = 0.0f;
+  int vs_cur = -112;  // the accumulators are in units of 2^(14 - vs_cur), which only grows
+
+  const size_t head_off = static_cast<size_t>(g) * kHd;
+  // this thread's share of a K tile and of a V tile, in flight while other
+  // tiles are multiplied.  Pre-split: pieces tid + 256 r of the record's
+  // arrays.  f16 cache: K pieces of dims 8 (tid % 32) .. +7 at positions
+  // tid / 32 + 8 r, and V dims 4 l .. 4 l + 3 of the eight positions of piece w.
+  typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
+  u32x4v kreg[4 * kParts], vreg[PRE ? 8 : 1];
+  u32x2v vpair[PRE ? 1 : 8];
+  // (f16 loads go through buffer descriptors that end at the chunk's last
+  // row: rows past it read as zero and need no address arithmetic; so does a
+  // tile past the end, whose descriptor is empty)
+  const int row_b = static_cast<int>(a.kv_stride * 2);
+  const int koff = (tid >> 5) * row_b + 16 * (tid & 31), voff = wide_vpos(w, 0) * row_b + 8 * l;
+  float ksr = 0.0f;
+  int vst = 0;  // PRE: the V tile's units are 2^vst
+  const size_t last_tile = (end - 1) / kMqTile;
+  auto tile_rsrc = [&](const void *cache, size_t t0) {
+    const size_t rows = t0 < end ? (end - t0 < kMqTile ? end - t0 : kMqTile) : 0;
+    const uint16_t *base = static_cast<const uint16_t *>(cache) + (rows ? t0 : 0) * a.kv_stride + head_off;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(base), 0,
+                                             rows ? static_cast<int>(rows - 1) * row_b + 2 * kHd : 0, 0x00020000);
+  };
+  auto fetch_k = [&](size_t t0) {
+    if constexpr (PRE) {
+      const size_t tile = t0 / kMqTile < last_tile ? t0 / kMqTile : last_tile, rec = tile * a.n_kv + g;
+      const u32x4v *src = reinterpret_cast<const u32x4v *>(a.rec) + rec * (4 * kWideArr / 8);
+#pragma unroll
+      for (int r = 0; r < 8; ++r) kreg[r] = src[kWideThreads * r + tid];
+      ksr = a.ks[rec * kMqTile + (tid & 31)];
+    } else {
+      const auto rsrc = tile_rsrc(a.kc, t0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        kreg[r] = __builtin_bit_cast(u32x4v, __builtin_amdgcn_raw_buffer_load_b128(rsrc, koff + 8 * r * row_b, 0, 0));
+    }
+  };
+  auto fetch_v = [&](size_t t0) {
+    if constexpr (PRE) {
+      const size_t tile = t0 / kMqTile < last_tile ? t0 / kMqTile : last_tile, rec = tile * a.n_kv + g;
+      const u32x4v *src = reinterpret_cast<const u32x4v *>(a.rec) + rec * (4 * kWideArr / 8) + 2 * kWideArr / 8;
+#pragma unroll
+      for (int r = 0; r < 8; ++r) vreg[r] = src[kWideThreads * r + tid];
+      vst = a.vsh[rec];
+    } else {
+      const auto rsrc = tile_rsrc(a.vc, t0);
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        vpair[j] = __builtin_bit_cast(u32x2v, __builtin_amdgcn_raw_buffer_load_b64(rsrc, voff + wide_vpos(0, j) * row_b, 0, 0));
+    }
+  };
+  // the stores of a K and a V tile, a few at a time
+  constexpr int kStageK = 4 * kParts, kStageV = PRE ? 8 : 4;
+  auto stage_k = [&](int buf, int r) {
+    const int at = PRE ? 8 * (tid + kWideThreads * r) : wide_k((tid >> 5) + 8 * r, tid & 31);
+    *reinterpret_cast<u32x4v *>(sT[0][buf] + at) = kreg[r];
+    if constexpr (PRE) {
+      if (r == 0) sKs[buf][tid & 31] = ksr;
+    }
+  };
+  auto stage_v = [&](int buf, int r) {
+    if constexpr (PRE) {
+      *reinterpret_cast<u32x4v *>(sT[1][buf] + 8 * (tid + kWideThreads * r)) = vreg[r];
+    } else {
+      // half r of each of the eight positions
+      u32x4v col;
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj)
+        col[jj] = __builtin_amdgcn_perm(vpair[2 * jj + 1][r >> 1], vpair[2 * jj][r >> 1],
+                                        (r & 1) ? 0x07060302u : 0x05040100u);
+      *reinterpret_cast<u32x4v *>(sT[1][buf] + wide_v(4 * l + r, w)) = col;
+    }
+  };
+  // lane addresses of the operand pieces: K k-steps differ in the XOR by s % 4
+  int ko[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) ko[s] = wide_k(r32, 2 * s + h);
+  const int vo = wide_v(r32, h);
+  // Operand pieces are read kAhead steps before their products: with one
+  // wave per SIMD nothing else covers the LDS latency.  The group of a step
+  // ends in a scheduling barrier, which keeps that distance and leaves the
+  // arithmetic given to the step beside its products.
+  constexpr int kAhead = 4;
+  half8 fr[kParts][kAhead];
+  auto read_k = [&](int buf, int s) {
+#pragma unroll
+    for (int k = 0; k < kParts; ++k)
+      fr[k][s % kAhead] = *reinterpret_cast<const half8 *>(
+          sT[0][buf] + k * kWideArr + ko[s & 3] + (s >> 2) * (4 * 64 * 8));
+  };
+  auto read_v = [&](int buf, int s) {
+#pragma unroll
+    for (int k = 0; k < kParts; ++k)
+      fr[k][s % kAhead] = *reinterpret_cast<const half8 *>(sT[1][buf] + k * kWideArr + vo + (2 * (s & 7) + (s >> 3)) * (64 * 8));
+  };
+  // S^T = K' Q'^T of a staged tile: row r32, positions 8 (i / 4) + 4 h + i % 4;
+  // the small cross products in their own accumulator; beside(s) is the
+  // arithmetic that goes with step s, and V's first pieces of buffer vbuf
+  // are read at the end
+  f32x16 s0, s1;
+  auto scores = [&](int buf, int vbuf, auto &&beside) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s0[i] = s1[i] = 0.0f;
+#pragma unroll
+    for (int s = 0; s < kAhead; ++s) read_k(buf, s);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < 16; ++s) {
+      s0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[0][s % kAhead], qh[s], s0, 0, 0, 0);
+      s1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[0][s % kAhead], ql[s], s1, 0, 0, 0);
+      if constexpr (PRE) s1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[kParts - 1][s % kAhead], qh[s], s1, 0, 0, 0);
+      if (s + kAhead < 16)
+        read_k(buf, s + kAhead);
+      else
+        read_v(vbuf, s + kAhead - 16);
+      beside(s);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // unscaled and masked (causal limit of the row, the chunk's end), with the
+  // row's largest
+  const size_t seen = limit < end ? limit : end;
+  float sc[16];
+  float tmax;
+  int vis;
+  f32x4 kfac[PRE ? 4 : 1];
+  auto mask_begin = [&](size_t t0, int buf) {
+    vis = (seen > t0 ? static_cast<int>(seen - t0 < kMqTile ? seen - t0 : kMqTile) : 0) - 4 * h;
+    tmax = -INFINITY;
+    if constexpr (PRE) {
+#pragma unroll
+      for (int i4 = 0; i4 < 4; ++i4) kfac[i4] = *reinterpret_cast<const f32x4 *>(&sKs[buf][8 * i4 + 4 * h]);
+    }
+  };
+  // element i goes through unscale at step i and hide at step i + 1, so that
+  // a step's arithmetic is of two elements and not one serial chain
+  auto unscale = [&](int i) {
+    float x = s0[i] + s1[i];
+    if constexpr (PRE) x *= kfac[i >> 2][i & 3];
+    sc[i] = x * qunscale;
+  };
+  auto hide = [&](int i) {
+    sc[i] = 8 * (i >> 2) + (i & 3) < vis ? sc[i] : -INFINITY;
+    tmax = fmaxf(tmax, sc[i]);
+  };
+  // the running reference follows the maximum only when that has grown by
+  // more than ln 16, so the accumulators are seldom rescaled (p <= 16 then,
+  // and p * 2^11 fits f16)
+  float pscale = 2048.0f;
+  auto settle = [&]() {
+    tmax = pair_max(tmax);
+    const bool grow = tmax > run_m + 2.7725887f;
+    int vs = vs_cur;
+    if constexpr (PRE) {
+      // the tile's V is in units of 2^vst, the block's of 2^vs
+      vs = vst > vs_cur ? vst : vs_cur;
+      pscale = 2048.0f * pow2f(vst - vs);
+    }
+    if (__builtin_amdgcn_ballot_w64(grow) != 0 || vs != vs_cur) {
+      const float corr = grow ? exp_hw(run_m - tmax) : 1.0f;
+      run_l *= corr;
+      const float ocorr = PRE ? corr * pow2f(vs_cur - vs) : corr;
+      run_m = grow ? tmax : run_m;
+      vs_cur = vs;
+#pragma unroll
+      for (int dt = 0; dt < 8; ++dt) {
+        // the pins keep the accumulators where the products hold them, so the
+        // copies for these products stay inside this block
+        asm volatile("" : "+a"(o[dt]));
+        o[dt] = o[dt] * ocorr;
+        asm volatile("" : "+a"(o[dt]));
+      }
+    }
+  };
+
+  fetch_k(beg);
+  fetch_v(beg);
+#pragma unroll
+  for (int r = 0; r < kStageK; ++r) stage_k(0, r);
+#pragma unroll
+  for (int r = 0; r < kStageV; ++r) stage_v(0, r);
+  fetch_k(beg + kMqTile);
+#pragma unroll
+  for (int r = 0; r < kStageK; ++r) stage_k(1, r);
+  __syncthreads();
+  scores(0, 0, [](int) {});
+  mask_begin(beg, 0);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    unscale(i);
+    hide(i);
+  }
+  settle();
+  int buf = 0;
+  // Each pass multiplies K of the next tile while this tile's exponentials
+  // are taken, then V of this tile while the next tile's scores are masked:
+  // one wave per SIMD, so what overlaps has to come from one instruction
+  // stream.
+  for (size_t t0 = beg; t0 < end; t0 += kMqTile, buf ^= 1) {
+    fetch_k(t0 + 2 * kMqTile);
+    fetch_v(t0 + kMqTile);
+    __builtin_amdgcn_sched_barrier(0);
+    const float m_sub = run_m == -INFINITY ? 0.0f : run_m;  // every score is -inf then
+    float psum = 0.0f;
+    half8 ph[2], pl[2];
+    // e^(score - m) as exp_hw forms it, in stages a step apart: four elements
+    // are under way at a time, their chains side by side
+    float et[16], ee[16], ex[16];
+    auto exps = [&](int step) {
+      if (step < 16) {
+        const int k = step;
+        const float x = sc[k] - m_sub;
+        et[k] = x * kExpL2E;
+        ee[k] = __builtin_fmaf(x, kExpL2ELo, __builtin_fmaf(x, kExpL2E, -et[k]));
+      }
+      if (step >= 1 && step - 1 < 16) {
+        const int k = step - 1;
+        ex[k] = __builtin_amdgcn_exp2f(et[k]);
+        ee[k] = __builtin_fmaf(ee[k], kExpLn2, 1.0f);
+      }
+      if (step >= 2 && step - 2 < 16) {
+        const int k = step - 2;
+        ex[k] = et[k] == -INFINITY ? 0.0f : ex[k] * ee[k];
+        psum += ex[k];
+        ex[k] *= pscale;
+      }
+      if (step >= 3 && step - 3 < 16) {
+        const int k = step - 3;
+        _Float16 hi, lo;
+        split_hl(ex[k], hi, lo);
+        ph[k >> 3][k & 7] = hi;
+        pl[k >> 3][k & 7] = lo;
+      }
+    };
+    // (past the last tile these are scores of stale positions, not used)
+    scores(buf ^ 1, buf, exps);
+    mask_begin(t0 + kMqTile, buf ^ 1);
+    // O^T += V'^T P'^T, the first sixteen positions of every dim tile first
+#pragma unroll
+    for (int s = 0; s < 16; ++s) {
+      f32x16 &od = o[s & 7];
+      od = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[0][s % kAhead], ph[s >> 3], od, 0, 0, 0);
+      od = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[0][s % kAhead], pl[s >> 3], od, 0, 0, 0);
+      if constexpr (PRE) od = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[kParts - 1][s % kAhead], ph[s >> 3], od, 0, 0, 0);
+      if (s + kAhead < 16) read_v(buf, s + kAhead);
+      if (s < 3) exps(16 + s);
+      if (s == 3) run_l += pair_sum(psum);
+      if (s >= 1) unscale(s - 1);
+      if (s >= 2) hide(s - 2);
+      // the buffers written here were last read before the previous barrier
+      constexpr int kFirst = 16 - kStageK - kStageV;
+      if (s >= kFirst && s < kFirst + kStageK) stage_k(buf, s - kFirst);
+      if (s >= kFirst + kStageK) stage_v(buf ^ 1, s - kFirst - kStageK);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    unscale(15);
+    hide(14);
+    hide(15);
+    settle();
+    __syncthreads();
+  }
+  if (valid) {
+    const float u = PRE ? pow2f(vs_cur - 11) : 1.0f / 2048.0f;
+    const bool fin = a.out != nullptr;
+    f32x4 *dst = reinterpret_cast<f32x4 *>(
+        fin ? a.out + (static_cast<size_t>(qi) * a.n_head + head) * kHd : a.pacc + part * kHd);
+    if (!fin && h == 0) {
+      a.pm[part] = run_m;
+      a.pl[part] = run_l;
+    }
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt)
+#pragma unroll
+      for (int i4 = 0; i4 < 4; ++i4) {
+        f32x4 v = {o[dt][4 * i4], o[dt][4 * i4 + 1], o[dt][4 * i4 + 2], o[dt][4 * i4 + 3]};
+        v = v * u;
+        // the merge of one chunk: weight e^0 = 1, so (acc * 1) / (l * 1)
+        // (the merge's 0 + acc turns an exact -0 into +0; nothing else differs)
+        if (fin) v = v / run_l;
+        dst[8 * dt + 2 * i4 + h] = v;
+      }
+  }
+}
+
+__global__ __launch_bounds__(kWideThreads, 1) void attn_mq_wide_f16_kernel(MqArgs a) { mq_wide_body<false>(a); }
+
+// The f32 path over the records of attn_kv_record_kernel.
+__global__ __launch_bounds__(kWideThreads, 1) void attn_mq_wide_pre_kernel(MqArgs a) { mq_wide_body<true>(a); }
+
+// attn_kv_split_kernel's scales and splits in the wide form's layout: block
+// (tile, g) writes the tile's record of K hi, K lo, V hi, V lo, each 16 KB in
+// the order in which the multi-query block stages it (wide_k, wide_v), so
+// staging is a linear copy.  The record is put together in LDS: its pieces
+// are 16 bytes at 512-byte strides, and go to memory as whole lines.
+__global__ __launch_bounds__(256) void attn_kv_record_kernel(const float *kc, const float *vc,
+                                                             size_t n_pos, size_t kv_stride, int n_kv,
+                                                             uint16_t *rec, float *ks, int *vsh) {
+  __shared__ __attribute__((aligned(16))) _Float16 sT[4 * kWideArr];
+  __shared__ float sm[4];
+  const int tile = static_cast<int>(blockIdx.x) / n_kv, g = static_cast<int>(blockIdx.x) % n_kv;
+  const size_t p0 = static_cast<size_t>(tile) * kMqTile, head_off = static_cast<size_t>(g) * kHd;
+  const int tid = threadIdx.x, kpart = tid & 15;
+#pragma unroll
+  for (int pass = 0; pass < kMqTile / 16; ++pass) {
+    const int sp = 16 * pass + (tid >> 4);
+    const size_t p = p0 + sp;
+    const bool ok = p < n_pos;
+    const size_t off = p * kv_stride + head_off + 16 * kpart;
+    f32x4 x[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      x[k] = ok ? *reinterpret_cast<const f32x4 *>(kc + off + 4 * k) : f32x4{0.f, 0.f, 0.f, 0.f};
+    float km = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      km = fmaxf(km, fmaxf(fmaxf(fabsf(x[k].x), fabsf(x[k].y)), fmaxf(fabsf(x[k].z), fabsf(x[k].w))));
+    km = lane_group_reduce<16>(km, FMaxOp{});
+    const int kb = split_shift(km);
+    const float kf = ldexpf(1.0f, kb);
+#pragma unroll
+    for (int k2 = 0; k2 < 2; ++k2) {
+      half8 hv, lv;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        _Float16 h, lo;
+        split_hl(x[2 * k2 + (k >> 2)][k & 3] * kf, h, lo);
+        hv[k] = h;
+        lv[k] = lo;
+      }
+      const int at = wide_k(sp, 2 * kpart + k2);
+      *reinterpret_cast<half8 *>(sT + at) = hv;
+      *reinterpret_cast<half8 *>(sT + kWideArr + at) = lv;
+    }
+    if (kpart == 0) ks[static_cast<size_t>(blockIdx.x) * kMqTile + sp] = ldexpf(1.0f, -kb);
+  }
+  // V: dim tid of the tile's positions (past the cache's end, copies of
+  // its last row: finite values the kernel masks)
+  float v[kMqTile];
+  float vm = 0.0f;
+#pragma unroll
+  for (int i = 0; i < kMqTile; ++i) {
+    const size_t p = p0 + i < n_pos ? p0 + i : n_pos - 1;
+    v[i] = vc[p * kv_stride + head_off + tid];
+    vm = fmaxf(vm, fabsf(v[i]));
+  }
+  vm = wave_max(vm);
+  if ((tid & 63) == 0) sm[tid >> 6] = vm;
+  __syncthreads();
+  vm = fmaxf(fmaxf(sm[0], sm[1]), fmaxf(sm[2], sm[3]));
+  const int vst = v_shift(vm);
+  if (tid == 0) vsh[blockIdx.x] = vst;
+  const float vf = ldexpf(1.0f, -vst);
+#pragma unroll
+  for (int pp = 0; pp < 4; ++pp) {
+    half8 hv, lv;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      _Float16 h, lo;
+      split_hl(v[wide_vpos(pp, j)] * vf, h, lo);
+      hv[j] = h;
+      lv[j] = lo;
+    }
+    const int at = 2 * kWideArr + wide_v(tid, pp);
+    *reinterpret_cast<half8 *>(sT + at) = hv;
+    *reinterpret_cast<half8 *>(sT + kWideArr + at) = lv;
+  }
+  __syncthreads();
+  u32x4v *dst = reinterpret_cast<u32x4v *>(rec + static_cast<size_t>(blockIdx.x) * (4 * kWideArr)) + tid;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) dst[256 * r] = *reinterpret_cast<const u32x4v *>(sT + 8 * (tid + 256 * r));
+}
+
 template <int PB, bool VQ>
 __global__ __launch_bounds__(kMqThreads) void attn_mq_planar_kernel(MqArgs a, PlanarTables tb) {
   mq_body<false, PB, VQ>(a, tb.cent, tb.gc, tb.gs);
@@ -2051,9 +2571,37 @@ extern "C" int bh_attention(const float *q, size_t n_q, size_t pos0, const void 
     if (nb > 0x7fffffffu) return fail(BH_ERR_SHAPE, "attention: too many blocks");
     const dim3 grid(static_cast<unsigned>(nb));
     // an f32 cache read by many row tiles per kv head (a prefill) is split
-    // into f16 hi / lo once instead of in every block
+    // into f16 hi / lo once instead of in every block.  Blocks of eight and
+    // more position tiles take the 32-row form: its loop is faster (2.3 us a
+    // tile against 2.9 over an f16 cache) and its start and end cost 4 us
+    // more, q's fragments passing through LDS and the pipeline filling.
+    // Measured, 16-row / 32-row form, us a call with its q and k steps: 1 tile
+    // a block (16 queries at 1000, f16) 29.0 / 32.5, 3 (333 at 0) 48.4 / 51.5,
+    // 4 (22 at 4000) 38.7 / 40.5, 7 (64 at 4032) 47.7 / 47.6, 8 (512 at 0, f32)
+    // 78.3 / 77.1, 12 (200 at 2000, f32) 90.8 / 82.7, 15 (8 at 30000) 63.9 /
+    // 58.6, 35 (333 at 4000) 132.8 / 114.3, 64 (2048 at 0, f32) 304 / 264.
     const bool pre = !f16 && tiles_r >= kMqPreTiles;
-    if (pre) {
+    const bool wide = (f16 || pre) && per >= kWideMinTiles;
+    if (pre && wide) {
+      const size_t n_tiles = (n_max + kMqTile - 1) / kMqTile;
+      const size_t rec_b = n_tiles * n_kv * (4 * kWideArr) * 2;  // whole tiles (rows past the end padded)
+      const size_t ks_b = n_tiles * n_kv * kMqTile * 4;
+      uint8_t *base = static_cast<uint8_t *>(
+          device_scratch(rec_b + ks_b + n_tiles * n_kv * 4, kScratchKvSplit, st));
+      if (base == nullptr) return BH_ERR_HIP;
+      uint16_t *rec = reinterpret_cast<uint16_t *>(base);
+      float *ks = reinterpret_cast<float *>(base + rec_b);
+      int *vsh = reinterpret_cast<int *>(base + rec_b + ks_b);
+      BH_LAUNCH(attn_kv_record_kernel, static_cast<unsigned>(n_tiles * n_kv), 256, 0, st,
+                static_cast<const float *>(k_cache), static_cast<const float *>(v_cache), n_max,
+                kv_stride, static_cast<int>(n_kv), rec, ks, vsh);
+      m.rec = rec;
+      m.ks = ks;
+      m.vsh = vsh;
+      BH_LAUNCH(attn_mq_wide_pre_kernel, grid, kWideThreads, 0, st, m);
+    } else if (wide) {
+      BH_LAUNCH(attn_mq_wide_f16_kernel, grid, kWideThreads, 0, st, m);
+    } else if (pre) {
       const size_t n_tiles = (n_max + kMqTile - 1) / kMqTile;
       const size_t halves = n_max * kv_stride;  // per array
       const size_t kh_b = (halves * 2 + 255) / 256 * 256;

@@ -225,15 +225,15 @@ __device__ __forceinline__ float softplus(float x) {
 // error a few 1e-7 for x <= 0 (what a softmax feeds it), against expf's
 // ~1e-7; -inf gives exactly 0, NaN stays NaN.  Used where a kernel is bound
 // by the exponentials and the result only needs the reference's tolerance.
+constexpr float kExpL2E = 1.44269502162933349609375f;   // log2(e) rounded to f32
+constexpr float kExpL2ELo = 1.925963033500011e-08f;     // log2(e) - kExpL2E
+constexpr float kExpLn2 = 0.693147180559945309f;
 __device__ __forceinline__ float exp_hw(float x) {
-  constexpr float kL2E = 1.44269502162933349609375f;   // log2(e) rounded to f32
-  constexpr float kL2ELo = 1.925963033500011e-08f;     // log2(e) - kL2E
-  constexpr float kLn2 = 0.693147180559945309f;
-  const float t = x * kL2E;
-  float err = __builtin_fmaf(x, kL2E, -t);
-  err = __builtin_fmaf(x, kL2ELo, err);
+  const float t = x * kExpL2E;
+  float err = __builtin_fmaf(x, kExpL2E, -t);
+  err = __builtin_fmaf(x, kExpL2ELo, err);
   const float r = __builtin_amdgcn_exp2f(t);
-  return x == -INFINITY ? 0.0f : r * __builtin_fmaf(err, kLn2, 1.0f);
+  return x == -INFINITY ? 0.0f : r * __builtin_fmaf(err, kExpLn2, 1.0f);
 }
 
 // silu with the hardware exponential (exp_hw) and reciprocal: within a few

@@ -245,3 +245,46 @@ def test_attention_presplit_tile_scales(bh, oracle, synth, dev):
     err = rel_err(got, ref)
     _say("  rel", err)
     assert err <= TOL
+
+
+@pytest.mark.parametrize("n_q,pos0,f16,span", [
+    (8, 1785, True, 0.0),    # 48 rows (two waves of four); the last chunk is one position
+    (8, 1816, True, 0.0),    # whole tiles only
+    (11, 1790, True, 0.0),   # 66 rows: a wave of two rows
+    (22, 1000, True, 0.0),   # 132 rows: a second row tile of four rows; a 30-position last tile
+    (64, 700, True, 32.0),   # scores that rise with the position: the reference moves many times
+    (8, 1000, True, 0.0),    # four tiles a block: the 16-row form
+    (256, 0, False, 0.0),    # a pre-split f32 cache, causal from position 0, one chunk
+    (171, 86, False, 32.0),  # its last tile holds one position
+    (172, 90, False, 64.0),  # each tile's scores far above the last one's
+    (171, 30, False, 0.0),   # seven tiles a block: the 16-row form
+])
+def test_attention_wide_rows(bh, oracle, synth, dev, n_q, pos0, f16, span):
+    """The 32-row matrix-core form (blocks of eight and more position tiles
+    over f16 caches and f32 caches split beforehand; 32 kv heads, so that few
+    positions make such blocks) at the edges of its row and position tiles, and with keys whose scores
+    climb by `span` nats from the first position to the last, so that the
+    running reference and the accumulators move many times.  A score of s
+    nats is rounded to s * 2^-24 at best, which is the relative error of its
+    probability, times the few roundings of its sum: centred, |s| <= 42, and
+    the oracle is within 6e-6 of 64-bit arithmetic on these inputs (at the
+    uncentred |s| of 390 it is 1e-4 away, past TOL by itself)."""
+    n_head, n_kv, hd = 192, 32, 256
+    _say("attention wide rows", n_q, pos0, "f16" if f16 else "f32", span)
+    q, kc, vc = _case(synth, n_q, pos0, n_head, n_kv, hd, 1500 + n_q + pos0, qscale=1.0)
+    if span:
+        # q and k share a direction: a score is that of the position alone
+        # plus noise of unit size
+        u = np.float32(1.0 / np.sqrt(hd))
+        q += u * np.float32(16.0)
+        n = pos0 + n_q
+        ramp = (np.arange(n, dtype=np.float32) / np.float32(n - 1) - np.float32(0.5)) * np.float32(span)
+        kc = (kc + ramp[:, None] * u).astype(np.float32)
+    if f16:
+        kc = kc.astype(np.float16).view(np.uint16)
+        vc = vc.astype(np.float16).view(np.uint16)
+    ref = oracle.attention(q, pos0, kc, vc, n_kv)
+    got = _run(bh, dev, q, pos0, kc, vc, n_kv)
+    err = rel_err(got, ref)
+    _say("  rel", err)
+    assert err <= TOL
