@@ -385,8 +385,7 @@ def wl_pq2_matmul(bh, synth, dev, stream, n_rows, ne0, n_tok):
 
 def measure_mm(name, n_rows, ne0, n_tok, bh, synth, dev, stream, steps, warmup):
     """A product entry: HBM GB/s as every entry, plus useful TFLOP/s (2 flops
-    per weight and token) against the dense f16 MFMA peak; the x side runs
-    as two f16 MFMAs (hi, lo), so half that peak is the useful ceiling."""
+    per weight and token) against the dense f16 MFMA peak."""
     rec = measure(name, wl_pq2_matmul(bh, synth, dev, stream, n_rows, ne0, n_tok), steps,
                   warmup, stream)
     tflops = 2.0 * n_tok * n_rows * ne0 / (rec["ms"] * 1e-3) / 1e12

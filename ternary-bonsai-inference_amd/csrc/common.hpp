@@ -51,7 +51,7 @@ inline int pow2ceil(size_t v) {
 // capturing is refused (it would allocate inside the capture).  Returns
 // nullptr with the status recorded on failure.
 constexpr int kScratchSoftmax = 0;  // split-row softmax partials
-constexpr int kScratchMatmul = 1;   // PQ2_0 product: f16 x fragments, token scales
+constexpr int kScratchMatmul = 1;   // PQ2_0 product: x fragments and factors, unpacked rows, partial sums
 constexpr int kScratchAttention = 2;  // attention: chunk partials or probabilities
 constexpr int kScratchGather = 3;     // gather + RMSNorm: the row scales
 constexpr int kScratchGdn = 4;        // gated delta-net chunks: prepared matrices
