@@ -143,7 +143,7 @@ __host__ __device__ inline SeqUnits seq_units(int es, float x) {
 struct SeqStep {
   float s;        // the sum after the step
   uint32_t left;  // additions still to do
-  bool whole;     // all n stayed in the binade of s: s + n m units
+  bool whole;     // all n stayed in the binade of s: s + n m units, below its upper end
 };
 
 // Applies the run's steps that stay in the binade of the sum with bits sb,
@@ -169,7 +169,9 @@ __host__ __device__ inline SeqStep seq_step(uint32_t sb, float x, uint32_t n, co
   SeqStep r;
   r.s = more ? run + x : run;
   r.left = (special && sb != 0u) || !more ? 0u : n - k - 1u;
-  r.whole = !more;
+  // a last step rounded up onto the binade's upper end is done, but what
+  // follows it needs the next binade's units
+  r.whole = !more && (seq_f2u(run) ^ sb) < (1u << 23);
   return r;
 }
 

@@ -75,6 +75,40 @@ float by_turns(const float *x, const uint32_t *runs, int n_runs, int lanes, int 
   return s;
 }
 
+// A row whose second run's last addition lands exactly on the upper end of the
+// sum's binade (a rounded-up step: m = q + 1 divides the gap), with more runs
+// behind it, which have to be added in the next binade's units.  Random rows
+// land about once in a million.  Returns the number of blocks.
+int landing_row(float *x, uint32_t *n) {
+  for (;;) {
+    const uint32_t e = 3 + below(24);
+    const float d0 = half_val((e << 10) | below(1024));
+    x[0] = d0 * d0;
+    n[0] = 1 + below(100);
+    volatile float s = 0.0f;
+    for (uint32_t i = 0; i < n[0]; ++i) s = s + x[0];
+    const uint32_t sb = bh::seq_f2u(s);
+    const uint32_t gap = (1u << 24) - ((sb & 0x7fffffu) | 0x800000u);
+    for (int tries = 0; tries < 400; ++tries) {
+      const uint32_t down = below(6);
+      if (e < 1 + down) continue;
+      const float d = half_val(((e - down) << 10) | below(1024));
+      x[1] = d * d;
+      const bh::SeqUnits u = bh::seq_units(static_cast<int>(sb >> 23), x[1]);
+      if (u.m != u.q + 1 || u.tie || gap % u.m != 0 || gap / u.m > 128) continue;
+      n[1] = gap / u.m;
+      const int nblk = 3 + static_cast<int>(below(38));
+      for (int b = 2; b < nblk; ++b) {
+        const uint32_t de = below(6);
+        const float db = half_val(((e > de ? e - de : 1) << 10) | below(1024));
+        x[b] = db * db;
+        n[b] = below(129);
+      }
+      return nblk;
+    }
+  }
+}
+
 }  // namespace
 
 int main() {
@@ -113,6 +147,38 @@ int main() {
       if (bh::seq_f2u(got) != bh::seq_f2u(loop)) {
         if (fail < 10)
           std::printf("MISMATCH row %d kind %d lanes %d: loop %08x turns %08x\n", it, kind, lanes,
+                      bh::seq_f2u(loop), bh::seq_f2u(got));
+        ++fail;
+      }
+      ++rows;
+    }
+  }
+  {  // two such rows as they were found: 1 + 124 + 77 and 40-block data's first six runs
+    const float d0 = half_val(0x3c45u), d1 = half_val(0x2d55u);
+    const float xa[3] = {d0 * d0, d1 * d1, d1 * d1};
+    const uint32_t na[3] = {1, 124, 77};
+    const float xb[6] = {0.0879898667f, 0.00947723165f, 1.09186172f, 0.109112799f, 7.55140209e-05f, 0.342179298f};
+    const uint32_t nb[6] = {118, 83, 100, 70, 85, 75};
+    int turns = 0;
+    const float a = by_turns(xa, na, 3, 64, turns), b = by_turns(xb, nb, 6, 64, turns);
+    if (a != 2.53446317f || b != 153.663376f) {
+      std::printf("MISMATCH literal rows: %.9g %.9g\n", a, b);
+      ++fail;
+    }
+  }
+  for (int it = 0; it < 1000; ++it) {
+    float x[160];
+    uint32_t n[160];
+    const int nblk = landing_row(x, n);
+    volatile float loop = 0.0f;
+    for (int b = 0; b < nblk; ++b)
+      for (uint32_t i = 0; i < n[b]; ++i) loop = loop + x[b];
+    for (int lanes : {64, 7}) {
+      int turns = 0;
+      const float got = by_turns(x, n, nblk, lanes, turns);
+      if (bh::seq_f2u(got) != bh::seq_f2u(loop)) {
+        if (fail < 10)
+          std::printf("MISMATCH landing row %d lanes %d: loop %08x turns %08x\n", it, lanes,
                       bh::seq_f2u(loop), bh::seq_f2u(got));
         ++fail;
       }

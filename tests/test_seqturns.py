@@ -57,3 +57,62 @@ def test_gather_rms_row_kernel(bh, oracle, dev, ne0, n_ids):
     assert np.array_equal(ge.view(np.uint32), ref_e.view(np.uint32))
     assert np.array_equal(gn[finite].view(np.uint32), ref_n[finite].view(np.uint32))
     assert np.array_equal(np.isnan(gn), np.isnan(ref_n))
+
+
+def _landing_rows(n_rows, nblk, seed):
+    """Scale bits and counts of codes other than 1 of rows whose second run
+    ends exactly on the upper end of the sum's binade: its square is rounded
+    up to m units of the sum, and m divides the units left in the binade."""
+    rng = np.random.default_rng(seed)
+    half = np.arange(0x7c00, dtype=np.uint16).view(np.float16).astype(np.float32)
+    scales = np.zeros((n_rows, nblk), np.uint16)
+    runs = np.zeros((n_rows, nblk), np.int64)
+    scales[0, :3], runs[0, :3] = (0x3c45, 0x2d55, 0x2d55), (1, 124, 77)
+    r = 1
+    while r < n_rows:
+        e = int(rng.integers(9, 18))
+        h0, n0 = (e << 10) | int(rng.integers(1024)), int(rng.integers(1, 101))
+        s = np.float32(0)
+        for _ in range(n0):
+            s = s + half[h0] * half[h0]
+        unit = np.float64(np.spacing(s))
+        gap = int((2.0 ** (np.floor(np.log2(np.float64(s))) + 1) - np.float64(s)) / unit)
+        cand = np.arange((e - 6) << 10, (e + 1) << 10)
+        xu = np.float64(half[cand] * half[cand]) / unit
+        m = np.rint(xu).astype(np.int64)
+        ok = (m == np.floor(xu) + 1) & (xu - np.floor(xu) != 0.5)
+        ok &= (gap % np.maximum(m, 1) == 0) & (gap <= 128 * m)
+        if not ok.any():
+            continue
+        i = int(rng.choice(np.flatnonzero(ok)))
+        scales[r, :2], runs[r, :2] = (h0, cand[i]), (n0, gap // int(m[i]))
+        scales[r, 2:] = ((e - rng.integers(0, 6, nblk - 2)) << 10) | rng.integers(0, 1024, nblk - 2)
+        runs[r, 2:] = rng.integers(0, 129, nblk - 2)
+        r += 1
+    return scales, runs
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nblk", [4, 40])
+def test_gather_rms_run_ends_on_binade(bh, oracle, dev, nblk):
+    """Rows whose runs end exactly on a power of two, which their next runs
+    have to leave in the next binade's units: bit for bit in a short batch (the
+    sum by turns) and in a long one (the sum walked a lane per row)."""
+    import torch
+    rows, ne0 = 64, nblk * 128
+    scales, runs = _landing_rows(rows, nblk, 11 + nblk)
+    codes = np.ones((rows, nblk, 128), np.uint8)
+    codes[np.arange(128) < runs[..., None]] = 2
+    codes = codes.reshape(rows, nblk, 32, 4)
+    table = np.empty((rows, nblk, 34), np.uint8)
+    table[..., 0], table[..., 1] = scales & 0xff, scales >> 8
+    table[..., 2:] = codes[..., 0] | codes[..., 1] << 2 | codes[..., 2] << 4 | codes[..., 3] << 6
+    table = table.reshape(rows, nblk * 34)
+    w = np.ones(ne0, np.float32)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)  # noqa: E731
+    for n_ids in (rows, 16 * torch.cuda.get_device_properties(0).multi_processor_count):
+        ids = (np.arange(n_ids) % rows).astype(np.uint32)
+        _, n = bh.pq2_embed_gather(t(table), ne0, rows, t(ids), w=t(w), eps=1e-6)
+        _, ref = oracle.embed_gather(table, ne0, rows, ids[:rows], w, 1e-6)
+        got = n.cpu().numpy().reshape(-1, rows, ne0)
+        assert np.array_equal(got.view(np.uint32), np.broadcast_to(ref.view(np.uint32), got.shape))
