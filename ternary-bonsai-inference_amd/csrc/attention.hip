@@ -1892,6 +1892,7 @@ __device__ __forceinline__ void mq_wide_body(const MqArgs &a) {
     hide(i);
   }
   settle();
+  __syncthreads();  // the first pass below writes K buffer 0 and its factors, which were read here
   int buf = 0;
   // Each pass multiplies K of the next tile while this tile's exponentials
   // are taken, then V of this tile while the next tile's scores are masked:

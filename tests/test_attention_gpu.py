@@ -288,3 +288,32 @@ def test_attention_wide_rows(bh, oracle, synth, dev, n_q, pos0, f16, span):
     err = rel_err(got, ref)
     _say("  rel", err)
     assert err <= TOL
+
+
+@pytest.mark.parametrize("n_q,pos0,f16", [(22, 1100, True), (256, 0, False)])
+def test_attention_wide_rows_first_tile(bh, oracle, synth, dev, n_q, pos0, f16):
+    """The 32-row form's first staged tile is read by every wave before the
+    third takes its place: most of each row's weight is on the first tile of
+    its first chunk and keys of opposite sign stand two tiles later, so a
+    wave that saw those instead would be far off; the same bits in ten calls
+    of a full grid."""
+    import torch
+    n_head, n_kv, hd = 192, 32, 256
+    _say("attention first tile", n_q, pos0, "f16" if f16 else "f32")
+    q, kc, vc = _case(synth, n_q, pos0, n_head, n_kv, hd, 77 + n_q, qscale=1.0)
+    u = np.float32(1.0 / np.sqrt(hd))
+    q += u * np.float32(16.0)
+    kc = kc.astype(np.float32)
+    kc[:32] += u * np.float32(8.0)
+    kc[64:96] -= u * np.float32(8.0)
+    if f16:
+        kc = kc.astype(np.float16).view(np.uint16)
+        vc = vc.astype(np.float16).view(np.uint16)
+    ref = oracle.attention(q, pos0, kc, vc, n_kv)
+    tq, tk, tv = _t(q, dev), _t(kc, dev), _t(vc, dev)
+    first = bh.attention(tq, pos0, tk, tv, n_kv)
+    for _ in range(9):
+        assert torch.equal(bh.attention(tq, pos0, tk, tv, n_kv), first)
+    err = rel_err(_h(first), ref)
+    _say("  rel", err)
+    assert err <= TOL
