@@ -1845,23 +1845,26 @@ __device__ __forceinline__ void mq_wide_body(const MqArgs &a) {
     tmax = fmaxf(tmax, sc[i]);
   };
   // the running reference follows the maximum only when that has grown by
-  // more than ln 16, so the accumulators are seldom rescaled (p <= 16 then,
-  // and p * 2^11 fits f16)
-  float pscale = 2048.0f;
+  // more than ln 3.9, so that not every tile rescales the accumulators; p <=
+  // 3.9 then, and p * 2^14 fits f16.  That is the 16-row form's unit: a small p
+  // behind an early maximum keeps its bits (at ln 16 and 2^11, 2^-18 of a
+  // flat tail's p = 2^-18 was lost, and 333 queries at 4000 took 110 us for 115)
+  float pscale = 16384.0f;
   auto settle = [&]() {
     tmax = pair_max(tmax);
-    const bool grow = tmax > run_m + 2.7725887f;
     int vs = vs_cur;
     if constexpr (PRE) {
       // the tile's V is in units of 2^vst, the block's of 2^vs
       vs = vst > vs_cur ? vst : vs_cur;
-      pscale = 2048.0f * pow2f(vst - vs);
+      pscale = 16384.0f * pow2f(vst - vs);
     }
-    if (__builtin_amdgcn_ballot_w64(grow) != 0 || vs != vs_cur) {
-      const float corr = grow ? exp_hw(run_m - tmax) : 1.0f;
+    if (__builtin_amdgcn_ballot_w64(tmax > run_m + 1.3609766f) != 0 || vs != vs_cur) {
+      // every row of the wave moves along: few reach the line by themselves later
+      const float m = fmaxf(run_m, tmax);
+      const float corr = m > run_m ? exp_hw(run_m - m) : 1.0f;
       run_l *= corr;
       const float ocorr = PRE ? corr * pow2f(vs_cur - vs) : corr;
-      run_m = grow ? tmax : run_m;
+      run_m = m;
       vs_cur = vs;
 #pragma unroll
       for (int dt = 0; dt < 8; ++dt) {
@@ -1962,7 +1965,7 @@ __device__ __forceinline__ void mq_wide_body(const MqArgs &a) {
     __syncthreads();
   }
   if (valid) {
-    const float u = PRE ? pow2f(vs_cur - 11) : 1.0f / 2048.0f;
+    const float u = PRE ? pow2f(vs_cur - 14) : 1.0f / 16384.0f;
     const bool fin = a.out != nullptr;
     f32x4 *dst = reinterpret_cast<f32x4 *>(
         fin ? a.out + (static_cast<size_t>(qi) * a.n_head + head) * kHd : a.pacc + part * kHd);

@@ -317,3 +317,35 @@ def test_attention_wide_rows_first_tile(bh, oracle, synth, dev, n_q, pos0, f16):
     err = rel_err(_h(first), ref)
     _say("  rel", err)
     assert err <= TOL
+
+
+@pytest.mark.parametrize("f16", [True, False])
+def test_attention_wide_rows_sink_and_flat_tail(bh, dev, f16):
+    """An early position that takes nearly all of a row's weight but holds a
+    zero value, and a flat tail behind it, whose probabilities of 2^-15 to
+    2^-19 are all rounded the same way.  In units of 2^-14 a probability p
+    splits into two f16 with an error of 2^-25 at most: 2^-39 / p, 2^-20 of it
+    at the smallest p here.  The eight tiles are 32 products, each of which
+    rounds an f32 sum once: 2^-24 each at most; exponential, row sum and
+    division are 8 more.  Scores are exact (multiples of 2^-8), the reference
+    is in 64 bits."""
+    import torch
+    n, n_head, n_kv, hd = 256, 192, 32, 256
+    rng = np.random.default_rng(5)
+    delta = np.round(rng.uniform(15, 19, (n, n_head)) * np.log(2.0) * 256) / 256
+    q = np.zeros((n, n_head, hd), np.float32)
+    q[..., 0] = 16 * delta
+    k = np.zeros((n, n_kv * hd), np.float32)
+    k[0, ::hd] = 1.0
+    vals = (1.0 + rng.integers(0, 1024, n_kv * hd) / 1024).astype(np.float32)
+    v = np.tile(vals, (n, 1))
+    v[0] = 0.0
+    cache = (lambda a: torch.from_numpy(a).to(dev).to(torch.float16).view(torch.int16)) if f16 else \
+        (lambda a: torch.from_numpy(a).to(dev))
+    got = _h(bh.attention(_t(q, dev), 0, cache(k), cache(v), n_kv)).reshape(n, n_head, hd)
+    p = np.exp(-delta)
+    tail = np.arange(n)[:, None] * p  # row i sees i positions of the tail
+    ref = (tail / (1.0 + tail))[..., None] * np.repeat(vals.reshape(n_kv, hd), n_head // n_kv, axis=0)
+    rel = np.abs(got[1:] / ref[1:] - 1.0).max()
+    _say("sink and tail", "f16" if f16 else "f32", rel)
+    assert rel <= 2.0 ** -20 + 40 * 2.0 ** -24
