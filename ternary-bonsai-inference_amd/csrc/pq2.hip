@@ -24,11 +24,12 @@
 // d*d as many times as it has codes other than 1, a run that seqsum.hpp
 // evaluates exactly without its additions.  Up to 16 rows per CU one launch:
 // a workgroup per row, one wave taking the row's runs by turns (a lane per
-// block) under the embedding stores, then the norm row.  Its time is the
-// launch, the row's first touch and about 15 turns: T = 1 8.4 us, 256 11.5,
-// 2048 17.2 (5.0 TB/s of 86.7 MB); a chain of the 5120 additions, a lane per
-// row, took 22.7, 27.8 and 29.5.  Longer batches: two launches of flat
-// writers (below), the sums walked a lane per row under the stores.
+// block; code 3 adds 4 d*d, see wave_row_ss) under the embedding stores, then
+// the norm row.  Its time is the launch, the row's first touch and about 15
+// turns: T = 1 8.4 us, 256 11.5, 2048 17.2 (5.0 TB/s of 86.7 MB); a chain of
+// the 5120 additions, a lane per row, took 22.7, 27.8 and 29.5.  Longer
+// batches: two launches of flat writers (below), the sums walked a lane per
+// row under the stores.
 #include <hip/hip_runtime.h>
 
 #include <string>
@@ -94,15 +95,56 @@ __device__ __forceinline__ uint32_t wave_prefix(uint32_t v) {
   return v;
 }
 
+// LDS of a wave that adds blocks weight by weight: the window's codes, eight
+// words a block, and one block's squares.
+struct HandLds {
+  uint32_t codes[64 * 8];
+  float sq[128];
+};
+
+// Adds the `valid` squares of block f of the window, whose scale bits are h, to
+// s in order, on one whole wave.  They pass through LDS, from where every lane
+// reads the same four at a time; squares past `valid` are +0, which leaves any
+// sum of squares as it is.
+__device__ __forceinline__ float wave_block_ss(float s, HandLds &m, int f, uint32_t h, int valid) {
+  const int lane = threadIdx.x & 63;
+  const float d = __uint_as_float(half_bits_to_f32_bits(h));
+  const bool finite = (h & 0x7c00u) != 0x7c00u;
+#pragma unroll
+  for (int j = lane; j < 128; j += 64) {
+    const float v = pq2_weight((m.codes[8 * f + (j >> 4)] >> (2 * (j & 15))) & 3u, d, finite);
+    m.sq[j] = j < valid ? v * v : 0.0f;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  const float4 *q4 = reinterpret_cast<const float4 *>(m.sq);
+#pragma unroll 8
+  for (int j = 0; j < 32; ++j) {
+    const float4 q = q4[j];
+    s += q.x;  // src/kernels.rs:65-68
+    s += q.y;
+    s += q.z;
+    s += q.w;
+  }
+  return s;
+}
+
 // The reference's sequential f32 sum of squares of the packed row, bit for
-// bit, on one whole wave.
-__device__ __forceinline__ float wave_row_ss(const uint8_t *row, int ne0, int nblk) {
+// bit, on one whole wave.  A block with code 3 holds squares of d d and of 4 d d;
+// it is added in closed form where it stays in the sum's binade and weight by
+// weight where not (a fifth of the blocks of four codes; a block of a
+// non-finite scale always).  Rows of four codes, T = 1 / 256 / 2048: 11.8 / 15.5
+// / 20.3 us, against 9.6 / 12.4 / 18.7 for three codes and 23.0 / 27.7 / 30.4 by
+// a chain of all 5120 additions; with every block of code 3 weight by weight
+// 29.5 / 31.1 / 39.0.
+__device__ __forceinline__ float wave_row_ss(const uint8_t *row, int ne0, int nblk, HandLds &hl) {
   const int lane = threadIdx.x & 63;
   float s = 0.0f;
   for (int b0 = 0; b0 < nblk; b0 += 64) {
     const int b = b0 + lane;
     float x = 0.0f;
-    uint32_t n = 0, by_hand = 0;
+    uint32_t n = 0, n4 = 0, h = 0;  // squares of d d and of 4 d d still to add
+    bool finite = true;
     if (b < nblk) {
       // the block's 34 bytes as eight aligned words and a halfword
       const bool even = (b & 1) == 0;
@@ -112,67 +154,83 @@ __device__ __forceinline__ float wave_row_ss(const uint8_t *row, int ne0, int nb
       uint32_t dw[8];
 #pragma unroll
       for (int k = 0; k < 8; ++k) dw[k] = w32[k];
-      const uint32_t h = even ? (dw[0] & 0xffffu) : h16;
+      h = even ? (dw[0] & 0xffffu) : h16;
       const int valid = ne0 - b * 128 < 128 ? ne0 - b * 128 : 128;
-      uint32_t ones = 0, threes = 0;
+      uint32_t ones = 0, threes = 0, w[8];
 #pragma unroll
       for (int k = 0; k < 8; ++k) {  // 16 codes a word
         const uint32_t nx = k < 7 ? dw[k < 7 ? k + 1 : 0] : h16;
-        const uint32_t w = even ? ((dw[k] >> 16) | (nx << 16)) : dw[k];
+        w[k] = even ? ((dw[k] >> 16) | (nx << 16)) : dw[k];
         const int lo = valid - 16 * k;
         const uint32_t mask =
             lo >= 16 ? 0x55555555u : (lo <= 0 ? 0u : 0x55555555u & ((1u << (2 * lo)) - 1u));
-        const uint32_t t = w ^ 0x55555555u;  // code 1 -> 00
+        const uint32_t t = w[k] ^ 0x55555555u;  // code 1 -> 00
         ones += __popc(~(t | (t >> 1)) & mask);
-        threes |= w & (w >> 1) & mask;
+        threes += __popc(w[k] & (w[k] >> 1) & mask);
       }
       const float d = __uint_as_float(half_bits_to_f32_bits(h));
       x = d * d;
-      n = x != 0.0f ? static_cast<uint32_t>(valid) - ones : 0u;  // d = 0: squares of +0
-      // a square of 4 d d, or a non-finite scale: weight by weight
-      by_hand = threes != 0u || (h & 0x7c00u) == 0x7c00u;
-      if (by_hand) n = 1;
-    }
-    for (;;) {
-      const uint32_t sb = __builtin_amdgcn_readfirstlane(__float_as_uint(s));
-      const SeqUnits u = seq_units(static_cast<int>(sb >> 23), x);
-      const uint32_t inc = n != 0u && by_hand == 0u ? seq_units_added(n, u) : 0u;
-      const uint32_t upto = wave_prefix(inc);
-      const uint32_t start = sb + (upto - inc);
-      const SeqStep step = seq_step(start, x, n, u);
-      const uint64_t stay = __ballot(n != 0u && (by_hand != 0u || !step.whole));
-      if (stay == 0u) {
-        s = __uint_as_float(sb + __builtin_amdgcn_readlane(upto, 63));
-        break;
+      finite = (h & 0x7c00u) != 0x7c00u;
+      if (x != 0.0f) {  // d = 0: squares of +0
+        n = static_cast<uint32_t>(valid) - ones - threes;
+        n4 = threes;
       }
-      const int f = __builtin_ctzll(stay);
-      uint32_t left = 0;
-      if (__builtin_amdgcn_readlane(by_hand, f) != 0) {
-        // src/kernels.rs:65-68: lane j squares weights j and j + 64
-        s = __uint_as_float(__builtin_amdgcn_readlane(start, f));
-        const uint8_t *blk = row + static_cast<size_t>(b0 + f) * kPq2Block;
-        const uint32_t h = *reinterpret_cast<const uint16_t *>(blk);
-        const float sc = __uint_as_float(half_bits_to_f32_bits(h));
-        const bool finite = (h & 0x7c00u) != 0x7c00u;
-        const int valid = ne0 - (b0 + f) * 128 < 128 ? ne0 - (b0 + f) * 128 : 128;
-        const float v0 = pq2_weight((blk[2 + (lane >> 2)] >> ((lane & 3) * 2)) & 3u, sc, finite);
-        const float v1 = pq2_weight((blk[18 + (lane >> 2)] >> ((lane & 3) * 2)) & 3u, sc, finite);
-        const uint32_t q0 = __float_as_uint(v0 * v0), q1 = __float_as_uint(v1 * v1);
-        for (int j = 0; j < valid; ++j)
-          s += __uint_as_float(j < 64 ? __builtin_amdgcn_readlane(q0, j)
-                                      : __builtin_amdgcn_readlane(q1, j - 64));
-      } else {
-        s = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(step.s), f));
-        left = __builtin_amdgcn_readlane(step.left, f);
+      if (!finite || n4 != 0u) {
+        n = finite ? n : 1u;
+        uint4 *c = reinterpret_cast<uint4 *>(hl.codes + 8 * lane);
+        c[0] = make_uint4(w[0], w[1], w[2], w[3]);
+        c[1] = make_uint4(w[4], w[5], w[6], w[7]);
       }
-      n = lane < f ? 0u : (lane == f ? left : n);
     }
+    const uint64_t hand = __ballot(!finite || n4 != 0u);
+    // HAND: the window has blocks of code 3 or a non-finite scale
+    auto turns = [&](auto hand_c) {
+      constexpr bool HAND = decltype(hand_c)::value;
+      for (;;) {
+        const uint32_t sb = __builtin_amdgcn_readfirstlane(__float_as_uint(s));
+        const int es = static_cast<int>(sb >> 23);
+        const SeqUnits u = seq_units(es, x);
+        const SeqUnits u4 = HAND ? seq_units(es, 4.0f * x) : u;
+        const uint32_t inc =
+            HAND ? (finite ? seq_mixed_added(n, u, n4, u4) : 0u) : (n != 0u ? seq_units_added(n, u) : 0u);
+        const uint32_t upto = wave_prefix(inc);
+        const uint32_t start = sb + (upto - inc);
+        const SeqStep step = seq_step(start, x, n, u);
+        bool whole = n == 0u || step.whole;
+        if constexpr (HAND) {
+          if (n4 != 0u) whole = seq_mixed_whole(start, inc, n, u, n4, u4);
+          whole = whole && (finite || n == 0u);
+        }
+        const uint64_t stay = __ballot(!whole);
+        if (stay == 0u) {
+          s = __uint_as_float(sb + __builtin_amdgcn_readlane(upto, 63));
+          break;
+        }
+        const int f = __builtin_ctzll(stay);
+        uint32_t left = 0;
+        if (HAND && ((hand >> f) & 1u) != 0u) {
+          const int rest = ne0 - (b0 + f) * 128;
+          s = wave_block_ss(__uint_as_float(__builtin_amdgcn_readlane(start, f)), hl, f,
+                            __builtin_amdgcn_readlane(h, f), rest < 128 ? rest : 128);
+        } else {
+          s = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(step.s), f));
+          left = __builtin_amdgcn_readlane(step.left, f);
+        }
+        n = lane < f ? 0u : (lane == f ? left : n);
+        if constexpr (HAND) n4 = lane <= f ? 0u : n4;
+      }
+    };
+    if (hand != 0u)
+      turns(std::true_type{});
+    else
+      turns(std::false_type{});
   }
   return s;
 }
 
 __global__ __launch_bounds__(kRowThreads) void pq2_gather_row_kernel(GatherArgs a) {
   __shared__ float row_scale;
+  __shared__ __attribute__((aligned(16))) HandLds hand;
   const size_t t = blockIdx.x;
   const uint32_t id = a.ids[t];
   const int n4 = a.ne0 >> 2;
@@ -189,7 +247,7 @@ __global__ __launch_bounds__(kRowThreads) void pq2_gather_row_kernel(GatherArgs 
   const uint8_t *row = a.table + static_cast<size_t>(id) * a.row_bytes;
   if (threadIdx.x < 64) {
     __builtin_amdgcn_s_setprio(3);  // the other waves wait for this one
-    const float ss = wave_row_ss(row, a.ne0, a.row_bytes / kPq2Block);
+    const float ss = wave_row_ss(row, a.ne0, a.row_bytes / kPq2Block, hand);
     // src/kernels.rs:69-70: mean = ss / n; scale = 1 / sqrt(mean + eps)
     if (threadIdx.x == 0) row_scale = 1.0f / sqrtf(ss / static_cast<float>(a.ne0) + a.eps);
     __builtin_amdgcn_s_setprio(0);

@@ -190,13 +190,29 @@ __host__ __device__ inline uint32_t repeat_add_step_f32(float &s, float x, uint3
 // its start by an exclusive prefix sum, and applies all runs up to the first
 // that does not stay (it leaves the binade, or is a tie from an odd sum);
 // that run's own step then carries the sum on, and the next turn starts from
-// there.  A row of 40 blocks takes about 19 turns of some 500 cycles instead
-// of 55 dependent steps of some 900.  An increment is cut to seq_units_added's
+// there.  A row of 40 blocks of model-like scales takes about 15 turns of some
+// 500 cycles instead of 55 dependent steps of some 900.  An increment is cut to
 // 2^25: past the end of the binade, where later starts no longer matter, and
 // 64 of them fit 32 bits.
 __host__ __device__ inline uint32_t seq_units_added(uint32_t n, const SeqUnits &v) {
   const uint32_t inc = n * v.m;  // <= 256 * 2^24 only past the binade; n <= 128 fits 32 bits
   return inc < (1u << 25) ? inc : 1u << 25;
+}
+
+// A block whose squares are n1 times x and n4 times 4 x, in any order: n1 m1 +
+// n4 m4 units, if they end below the binade's end (then no addition leaves it)
+// and none is a tie, whose rounding would depend on the sum before it.
+// n1 + n4 <= 128.  Otherwise it is added square by square.
+__host__ __device__ inline uint32_t seq_mixed_added(uint32_t n1, const SeqUnits &v1, uint32_t n4,
+                                                    const SeqUnits &v4) {
+  const uint32_t inc = n1 * v1.m + n4 * v4.m;
+  return inc < (1u << 25) ? inc : 1u << 25;
+}
+__host__ __device__ inline bool seq_mixed_whole(uint32_t start, uint32_t inc, uint32_t n1,
+                                                const SeqUnits &v1, uint32_t n4, const SeqUnits &v4) {
+  const bool special = start - 1u >= 0x7f7fffffu;  // +0, inf or NaN
+  const bool tie = (v1.tie & (n1 != 0u)) | (v4.tie & (n4 != 0u));
+  return !special & !tie & (((start & 0x7fffffu) | 0x800000u) + inc < (1u << 24));
 }
 
 }  // namespace bh

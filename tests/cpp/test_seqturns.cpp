@@ -75,6 +75,41 @@ float by_turns(const float *x, const uint32_t *runs, int n_runs, int lanes, int 
   return s;
 }
 
+// Blocks of squares x and 4 x in a drawn order, a lane each, as a wave takes
+// them: in closed form where the block stays in the binade, square by square
+// (in its order) where it does not.
+struct Mixed {
+  float x;
+  uint32_t n1, n4;
+  uint64_t four[2];  // place j holds 4 x (of the first n1 + n4)
+};
+float add_in_order(float s, const Mixed &b) {
+  volatile float acc = s;
+  for (uint32_t j = 0; j < b.n1 + b.n4; ++j)
+    acc = acc + (((b.four[j >> 6] >> (j & 63)) & 1u) ? 4.0f * b.x : b.x);
+  return acc;
+}
+float mixed_by_turns(const Mixed *b, int n_blk, int &turns) {
+  float s = 0.0f;
+  for (int done = 0; done < n_blk;) {
+    ++turns;
+    const uint32_t sb = bh::seq_f2u(s);
+    const int es = static_cast<int>(sb >> 23);
+    uint32_t at = sb;
+    int l = done;
+    for (; l < n_blk; ++l) {
+      const bh::SeqUnits u = bh::seq_units(es, b[l].x), u4 = bh::seq_units(es, 4.0f * b[l].x);
+      const uint32_t inc = bh::seq_mixed_added(b[l].n1, u, b[l].n4, u4);
+      if (b[l].n1 + b[l].n4 != 0 && !bh::seq_mixed_whole(at, inc, b[l].n1, u, b[l].n4, u4)) break;
+      at += inc;
+    }
+    s = bh::seq_u2f(at);
+    if (l < n_blk) s = add_in_order(s, b[l++]);
+    done = l;
+  }
+  return s;
+}
+
 // A row whose second run's last addition lands exactly on the upper end of the
 // sum's binade (a rounded-up step: m = q + 1 divides the gap), with more runs
 // behind it, which have to be added in the next binade's units.  Random rows
@@ -185,6 +220,44 @@ int main() {
       ++rows;
     }
   }
+  long by_hand = 0, mixed_rows = 0;
+  for (int it = 0; it < 12000; ++it) {  // rows of blocks of two kinds of squares
+    Mixed b[64];
+    const uint32_t base = below(28);
+    const int nblk = 1 + static_cast<int>(below(64));
+    volatile float loop = 0.0f;
+    for (int l = 0; l < nblk; ++l) {
+      uint32_t h;
+      switch (it % 4) {
+        case 0: h = 1 + below(0x7bffu); break;                // any scale
+        case 1: h = (5 + below(20)) << 10; break;             // powers of two: ties
+        case 2: h = 0x3c00u + (below(4) << 8); break;         // whole sums, ends on binades
+        default: h = ((base + below(3)) << 10) | below(1024);  // a few binades
+      }
+      const float d = half_val(h);
+      b[l].x = d * d;
+      b[l].n1 = b[l].n4 = 0;
+      b[l].four[0] = b[l].four[1] = 0;
+      const uint32_t n = below(5) == 0 ? below(3) : below(129);
+      for (uint32_t j = 0; j < n; ++j) {
+        const bool four = below(3) == 0;
+        b[l].four[j >> 6] |= static_cast<uint64_t>(four) << (j & 63);
+        ++(four ? b[l].n4 : b[l].n1);
+      }
+      loop = add_in_order(loop, b[l]);
+    }
+    int turns = 0;
+    const float got = mixed_by_turns(b, nblk, turns);
+    if (it % 4 == 3) by_hand += turns - 1, mixed_rows += nblk;
+    if (bh::seq_f2u(got) != bh::seq_f2u(loop)) {
+      if (fail < 10)
+        std::printf("MISMATCH mixed row %d: loop %08x turns %08x\n", it, bh::seq_f2u(loop), bh::seq_f2u(got));
+      ++fail;
+    }
+    ++rows;
+  }
+  std::printf("mixed blocks of a few binades: %.2f of them by hand\n",
+              static_cast<double>(by_hand) / static_cast<double>(mixed_rows));
   std::printf("%ld rows, %d mismatches, %.1f turns a row of 40 blocks\n", rows, fail,
               static_cast<double>(turns40) / static_cast<double>(rows40));
   return fail != 0;

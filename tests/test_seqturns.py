@@ -33,7 +33,7 @@ def test_row_by_turns_matches_sequential_loop(tmp_path, rcp_ulp):
 def test_gather_rms_row_kernel(bh, oracle, dev, ne0, n_ids):
     """One workgroup per row: rows of 2 blocks, a partial last block on rows
     that start on 4 bytes only, exactly one window of 64 blocks and a second
-    one of 6, with code-3 blocks (added by hand), zero and non-finite scales
+    one of 6, with code-3 blocks (two squares; by hand at a binade's end), zero and non-finite scales
     among the runs; both outputs bit for bit where the row is finite."""
     import torch
     rng = np.random.default_rng(ne0 + n_ids)
@@ -116,3 +116,36 @@ def test_gather_rms_run_ends_on_binade(bh, oracle, dev, nblk):
         _, ref = oracle.embed_gather(table, ne0, rows, ids[:rows], w, 1e-6)
         got = n.cpu().numpy().reshape(-1, rows, ne0)
         assert np.array_equal(got.view(np.uint32), np.broadcast_to(ref.view(np.uint32), got.shape))
+
+
+@pytest.mark.gpu
+def test_gather_rms_code_3_rows_cost(bh, dev):
+    """Rows of four codes cost about what rows of three do (their blocks are
+    summed in closed form too, but for those that leave a binade): a table's
+    codes must not decide the call's time.  Weight by weight they took 30
+    times as long; six leaves room for the clock."""
+    import torch
+    g = torch.Generator(device=dev)
+    g.manual_seed(3)
+    rows, nblk = 64, 40
+    w = torch.ones(nblk * 128, device=dev)
+    ids = torch.arange(rows, device=dev, dtype=torch.int32)
+    us = {}
+    for top in (3, 4):
+        table = torch.randint(0, top, (rows, nblk, 34, 4), device=dev, generator=g, dtype=torch.uint8)
+        table = table[..., 0] | table[..., 1] << 2 | table[..., 2] << 4 | table[..., 3] << 6
+        d = (torch.randn((rows, nblk), device=dev, generator=g) * 0.02).abs().to(torch.float16)
+        table[..., :2] = d.view(torch.uint8).view(rows, nblk, 2)
+        table = table.contiguous().view(-1)
+        times = []
+        for _ in range(5):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(50):
+                bh.pq2_embed_gather(table, nblk * 128, rows, ids, w=w, eps=1e-6)
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b) * 20)
+        us[top] = min(times)
+    print(us, flush=True)
+    assert us[4] <= 6 * us[3]
