@@ -52,6 +52,7 @@
 
 #include "common.hpp"
 #include "pq2_mx.hpp"
+#include "pq2_mx_plan.hpp"
 
 namespace bh {
 namespace {
@@ -67,10 +68,10 @@ typedef float f16v __attribute__((ext_vector_type(16)));
 // lane with the A scale bytes of h = 0, 1; rounded up to whole 16 KB.
 constexpr int kXHi = 2 * kDigits * 1024;
 constexpr int kXScale = kXHi + 2 * kDigits * 512;
-constexpr int kXRec = 16384;
+constexpr int kXRec = kMxXRec;
 // weight record of one (32-row tile, 128-block): operand planes [h] of 64
 // lanes x 16 bytes; the f32 block scales stand in an array of their own.
-constexpr int kWRec = 2048;
+constexpr int kWRec = kMxWRec;
 
 // Column of a lane's 32 of a half that k-slot e stands for.
 __host__ __device__ constexpr int mx_column(int e) {
@@ -234,6 +235,7 @@ constexpr int kRT = 4;          // row tiles (of 32) of a wave
 constexpr int kWR = 4, kWT = 2;  // waves of a workgroup along rows and tokens
 constexpr int kThreads = 64 * kWR * kWT;
 constexpr int kPanelRows = 32 * kRT * kWR, kSetTok = 32 * kWT;
+static_assert(kPanelRows == kMxPanelRows && kSetTok == kMxSetTok, "the plan's tile");
 
 // Tile q of the walk: 8 row panels by token sets, so that the tiles of
 // neighbouring units share their panels' and sets' records in L2.
@@ -659,59 +661,6 @@ __global__ __launch_bounds__(256) void pq2_mx_raw_fold_kernel(RawArgs a) {
     if (t + k < a.n_tok) a.y[static_cast<size_t>(t + k) * a.n_rows + row] = o[k];
 }
 
-size_t round256(size_t v) { return (v + 255) / 256 * 256; }
-
-constexpr int kRawWaves = 8;
-
-// How a call is cut: the raw kernel with R row tiles a wave (R = 1, 2), or the
-// unpacked kernel (R = 0), each with its tiles' blocks in `split` parts, and
-// the time that this is expected to take.  The times were fitted to calls of
-// 16 to 2048 tokens on [17408 x 5120], [5120 x 17408] and [6144 x 5120]
-// (within about 15 %): a turn of two blocks takes a round of raw workgroups
-// 1.9 us (R = 1) or 2.9 us (R = 2), a block takes a round of unpacked ones 2.3
-// us; a round costs 4 us besides; unpacking runs at 1.3 TB/s of packed bytes;
-// parts cost a launch and their sums through memory.
-struct Plan {
-  int R;
-  size_t full, split;
-  double us;
-};
-
-void raw_plan(size_t n_rows, size_t tok_tiles, size_t nblk, Plan &best) {
-  const size_t slots = device_cu_count(), pairs = nblk / 2;
-  for (int R = 1; R <= 2; ++R) {
-    const size_t rows = 32 * kRawWaves * R;
-    const size_t tiles = (n_rows + rows - 1) / rows * tok_tiles;
-    for (size_t s = 1; s <= std::min<size_t>(pairs, 32); ++s) {
-      const double rounds = static_cast<double>((tiles * s + slots - 1) / slots);
-      const double turns = static_cast<double>((pairs + s - 1) / s);
-      double us = rounds * (turns * (R == 1 ? 1.9 : 2.9) + 4.0);
-      if (s > 1) us += 5.0 + static_cast<double>(tiles * s * rows * 32 * 8) / 3e6;
-      if (us < best.us) best = Plan{R, 0, s, us};
-    }
-  }
-}
-
-// Whole rounds of tiles over the CUs (one workgroup each), then the rest in
-// parts that fill shorter rounds.
-void gemm_plan(size_t n_rows, size_t n_tok, size_t nblk, Plan &best) {
-  const size_t slots = device_cu_count();
-  const size_t tiles = (n_rows + kPanelRows - 1) / kPanelRows * ((n_tok + kSetTok - 1) / kSetTok);
-  const size_t full = slots % 8 == 0 ? tiles / slots * slots : 0, rest = tiles - full;
-  const double base = static_cast<double>(n_rows * nblk * kBlkBytes) / 1.3e6 + 5.0 +
-                      static_cast<double>(full / slots) * (static_cast<double>(nblk) * 2.3 + 4.0);
-  if (rest == 0) {
-    if (base < best.us) best = Plan{0, full, 1, base};
-    return;
-  }
-  for (size_t s = 1; s <= std::min<size_t>(nblk / 2, 16); ++s) {
-    const double rounds = static_cast<double>((rest * s + slots - 1) / slots);
-    double us = base + rounds * (static_cast<double>((nblk + s - 1) / s) * 2.3 + 4.0);
-    if (s > 1) us += 5.0 + static_cast<double>(rest * s * kPanelRows * kSetTok * 8) / 3e6;
-    if (us < best.us) best = Plan{0, full, s, us};
-  }
-}
-
 int xprep(const float *x, size_t ne0, size_t n_tok, uint8_t *rec, hipStream_t st) {
   const size_t nblk = ne0 / 128;
   const XPrepArgs a{x, rec, static_cast<int>(ne0), static_cast<int>(n_tok), static_cast<int>(nblk),
@@ -722,17 +671,13 @@ int xprep(const float *x, size_t ne0, size_t n_tok, uint8_t *rec, hipStream_t st
 
 template <int R>
 int launch_raw(const uint8_t *w, size_t ne0, size_t n_rows, const float *x, size_t n_tok, float *y,
-               size_t split, hipStream_t st) {
-  constexpr int W = kRawWaves;
+               size_t split, char *scratch, const MxScratch &m, hipStream_t st) {
+  constexpr int W = kMxRawWaves;
   const size_t nblk = ne0 / 128, tok_tiles = (n_tok + 31) / 32;
   const size_t panels = (n_rows + 32 * W * R - 1) / (32 * W * R), tiles = panels * tok_tiles;
-  const size_t x_bytes = tok_tiles * nblk * kXRec;
-  const size_t p_bytes = split > 1 ? tiles * split * 32 * W * R * 32 * sizeof(float) : 0;
-  char *scratch = static_cast<char *>(device_scratch(x_bytes + p_bytes, kScratchMatmul, st));
-  if (scratch == nullptr) return BH_ERR_HIP;
   uint8_t *rec = reinterpret_cast<uint8_t *>(scratch);
   if (int e = xprep(x, ne0, n_tok, rec, st)) return e;
-  const RawArgs a{w, rec, y, reinterpret_cast<float4 *>(scratch + x_bytes), bh_pq2_row_bytes(ne0),
+  const RawArgs a{w, rec, y, reinterpret_cast<float4 *>(scratch + m.x), bh_pq2_row_bytes(ne0),
                   static_cast<int>(n_rows), static_cast<int>(n_tok), static_cast<int>(nblk),
                   static_cast<int>(tok_tiles), static_cast<int>(split)};
   constexpr int lds = 4 * kXRec + 32 * W * R * kRawPitch * 4;
@@ -748,40 +693,19 @@ int launch_raw(const uint8_t *w, size_t ne0, size_t n_rows, const float *x, size
 
 }  // namespace
 
-// Unpacked weights of one pass over the rows: bounds the scratch that a wide
-// matrix (the vocabulary) would take, at 68 bytes a row and block.
-constexpr size_t kUnpackBytes = 96 << 20;
-
 int pq2_mx_gemm(const uint8_t *w, size_t ne0, size_t n_rows, const float *x, size_t n_tok, float *y,
                 hipStream_t st) {
-  const size_t nblk = ne0 / 128, tok_tiles = (n_tok + 31) / 32;
-  Plan plan{1, 0, 1, 1e30};
-  raw_plan(n_rows, tok_tiles, nblk, plan);
-  gemm_plan(n_rows, n_tok, nblk, plan);
-  if (plan.R == 1) return launch_raw<1>(w, ne0, n_rows, x, n_tok, y, plan.split, st);
-  if (plan.R == 2) return launch_raw<2>(w, ne0, n_rows, x, n_tok, y, plan.split, st);
-
-  const size_t per_row = nblk * (kWRec / 32 + sizeof(float));
-  const size_t pass_rows = std::max<size_t>(1, kUnpackBytes / per_row / kPanelRows) * kPanelRows;
-  const size_t tsets = (n_tok + kSetTok - 1) / kSetTok;
-  auto pass_plan = [&](size_t rows) {
-    Plan p{0, 0, 1, 1e30};
-    gemm_plan(rows, n_tok, nblk, p);
-    return p;
-  };
-  auto part_bytes = [&](size_t rows, const Plan &p) {
-    const size_t rest = (rows + kPanelRows - 1) / kPanelRows * tsets - p.full;
-    return p.split > 1 ? rest * p.split * kPanelRows * kSetTok * sizeof(float) : 0;
-  };
-  const size_t rows0 = std::min(n_rows, pass_rows), last = n_rows % rows0 ? n_rows % rows0 : rows0;
-  const size_t tiles0 = (rows0 + 31) / 32;
-  const size_t x_bytes = tok_tiles * nblk * kXRec, w_bytes = tiles0 * nblk * kWRec;
-  const size_t d_bytes = round256(tiles0 * nblk * 32 * sizeof(float));
-  const size_t p_bytes =
-      std::max(part_bytes(rows0, pass_plan(rows0)), part_bytes(last, pass_plan(last)));
-  char *scratch =
-      static_cast<char *>(device_scratch(x_bytes + w_bytes + d_bytes + p_bytes, kScratchMatmul, st));
+  const size_t nblk = ne0 / 128, slots = device_cu_count();
+  const MxPlan plan = mx_plan(n_rows, n_tok, nblk, slots);
+  const MxScratch m = mx_scratch_of(plan, n_rows, n_tok, nblk, slots);
+  char *scratch = static_cast<char *>(
+      device_scratch(std::max(m.total(), mx_reserve_bytes(n_rows, n_tok, nblk)), kScratchMatmul, st));
   if (scratch == nullptr) return BH_ERR_HIP;
+  if (plan.R == 1) return launch_raw<1>(w, ne0, n_rows, x, n_tok, y, plan.split, scratch, m, st);
+  if (plan.R == 2) return launch_raw<2>(w, ne0, n_rows, x, n_tok, y, plan.split, scratch, m, st);
+
+  const size_t pass_rows = mx_pass_rows(nblk), tok_tiles = (n_tok + 31) / 32;
+  const size_t tsets = (n_tok + kSetTok - 1) / kSetTok;
   uint8_t *rec = reinterpret_cast<uint8_t *>(scratch);
   if (int e = xprep(x, ne0, n_tok, rec, st)) return e;
   constexpr int lds = 2 * kWT * kXRec;
@@ -792,16 +716,16 @@ int pq2_mx_gemm(const uint8_t *w, size_t ne0, size_t n_rows, const float *x, siz
   for (size_t r0 = 0; r0 < n_rows; r0 += pass_rows) {
     const size_t rows = std::min(n_rows - r0, pass_rows), row_tiles = (rows + 31) / 32;
     const size_t panels = (rows + kPanelRows - 1) / kPanelRows;
-    const Plan p = pass_plan(rows);
+    const MxPlan p = mx_pass_plan(rows, n_tok, nblk, slots);
     const size_t rest = panels * tsets - p.full;
     const size_t row_bytes = bh_pq2_row_bytes(ne0);
-    const WPrepArgs wa{w + r0 * row_bytes, rec + x_bytes,
-                       reinterpret_cast<float *>(scratch + x_bytes + w_bytes), row_bytes,
+    const WPrepArgs wa{w + r0 * row_bytes, rec + m.x,
+                       reinterpret_cast<float *>(scratch + m.x + m.w), row_bytes,
                        static_cast<int>(rows), static_cast<int>(nblk),
                        static_cast<int>((nblk + kWChunk - 1) / kWChunk)};
     BH_LAUNCH(pq2_mx_wprep_kernel, static_cast<unsigned>(row_tiles * wa.chunks), 256, 0, st, wa);
     const GemmArgs a{rec, wa.rec, wa.scale, y + r0,
-                     reinterpret_cast<float4 *>(scratch + x_bytes + w_bytes + d_bytes),
+                     reinterpret_cast<float4 *>(scratch + m.x + m.w + m.d),
                      static_cast<int>(rows), static_cast<int>(n_tok), static_cast<int>(nblk),
                      static_cast<int>(n_rows), static_cast<int>(row_tiles),
                      static_cast<int>(tok_tiles), static_cast<int>(panels), static_cast<int>(tsets),
