@@ -2589,7 +2589,9 @@ extern "C" int bh_attention(const float *q, size_t n_q, size_t pos0, const void 
     if (pre && wide) {
       const size_t n_tiles = (n_max + kMqTile - 1) / kMqTile;
       const size_t rec_b = n_tiles * n_kv * (4 * kWideArr) * 2;  // whole tiles (rows past the end padded)
-      const size_t ks_b = n_tiles * n_kv * kMqTile * 4;
+      // (rounded as below: no fewer bytes than the 16-row form's for these
+      // positions, so that a call of more queries prepares a capture of fewer)
+      const size_t ks_b = (n_tiles * n_kv * kMqTile * 4 + 255) / 256 * 256;
       uint8_t *base = static_cast<uint8_t *>(
           device_scratch(rec_b + ks_b + n_tiles * n_kv * 4, kScratchKvSplit, st));
       if (base == nullptr) return BH_ERR_HIP;

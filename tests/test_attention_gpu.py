@@ -349,3 +349,48 @@ def test_attention_wide_rows_sink_and_flat_tail(bh, dev, f16):
     rel = np.abs(got[1:] / ref[1:] - 1.0).max()
     _say("sink and tail", "f16" if f16 else "f32", rel)
     assert rel <= 2.0 ** -20 + 40 * 2.0 ** -24
+
+
+_SPLIT_CAPTURE_SCRIPT = r'''
+import sys
+import torch
+sys.path.insert(0, sys.argv[1])
+from conftest import load_bonsai
+bh = load_bonsai()
+dev = torch.device("cuda:0")
+n_head, n_kv, hd, n = 8, 1, 256, 32 * 223
+k, v = torch.randn((n, n_kv * hd), device=dev), torch.randn((n, n_kv * hd), device=dev)
+qs = {t: torch.randn((t, n_head, hd), device=dev) for t in (2000, 120)}
+s = torch.cuda.Stream(device=dev)
+torch.cuda.synchronize()
+bh.attention(qs[2000], n - 2000, k, v, n_kv, stream=s)
+torch.cuda.synchronize()
+out = torch.empty_like(qs[120])
+g = torch.cuda.CUDAGraph()
+with torch.cuda.graph(g, stream=s):
+    bh.attention(qs[120], n - 120, k, v, n_kv, out=out, stream=s)
+want = bh.attention(qs[120], n - 120, k, v, n_kv)
+torch.cuda.synchronize()
+for rep in range(3):
+    out.fill_(float("nan"))
+    torch.cuda.synchronize()
+    g.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(out, want), rep
+print("capture ok")
+'''
+
+
+def test_attention_split_scratch_of_fewer_queries(dev):
+    """Over the same positions of an f32 cache, a call of 2000 queries (the
+    32-row form's records) prepares the capture of 120 (the 16-row form's split
+    halves, 223 tiles of one kv head: sizes whose rounding differs).  Runs in a
+    fresh process so no earlier call has grown the scratch."""
+    import subprocess
+    import sys
+    from pathlib import Path
+    here = Path(__file__).resolve().parent
+    res = subprocess.run([sys.executable, "-c", _SPLIT_CAPTURE_SCRIPT, str(here)], capture_output=True,
+                         text=True, timeout=100)
+    print(res.stdout[-2000:], res.stderr[-2000:])
+    assert res.returncode == 0 and "capture ok" in res.stdout
