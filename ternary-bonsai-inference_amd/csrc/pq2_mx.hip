@@ -9,12 +9,15 @@
 // k-slots of B:
 //   B = weights: the values code - 1 in {-1, 0, 1, 2}, halved, are exact in
 //       e2m1, so a block is multiplied as it is and the sum needs no
-//       correction for the code's offset (a weight of 0 adds exactly 0,
-//       whatever the size of its x);
+//       correction for the code's offset (a weight of 0 adds exactly 0, though
+//       a large x there coarsens the step of its group's other columns);
 //   A = x: each 32 columns of a token are scaled by the power of two that
 //       puts their largest |x| in [2^23, 2^24), rounded to integers X and
 //       written as five signed base-32 digits (-16 .. 16, exact in e2m3 as
-//       digit / 8): 24 significant bits, what f32 itself holds.  The group's
+//       digit / 8): a step of 2^-24 of the power of two above the group's
+//       largest |x|, which is 24 bits for that one (what f32 itself holds) and
+//       k fewer for a column 2^-k as large (the integer form: 22 bits of the
+//       largest of 128 columns; the f16 form: 22 of each column).  The group's
 //       power of two is the A scale, the digit's 2^(5 j) the B scale, so all
 //       ten products of a 128-block (two k halves, five digits) accumulate
 //       into one f32 tile and leave x in its own units;

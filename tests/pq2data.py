@@ -95,3 +95,23 @@ def decoded(payload: np.ndarray, ne0: int, n_rows: int, base_row: int = 0) -> np
     codes = np.stack([(qs >> (2 * k)) & 3 for k in range(4)], axis=-1).reshape(n_rows, nblk, 128)
     w = (codes.astype(np.float64) - 1.0) * scales[:, :, None]
     return w.reshape(n_rows, nblk * 128)[:, :ne0]
+
+
+# (ne0, n_rows, n_tok) of block-scaled products at the edges of their tiles and
+# how csrc/pq2_mx_plan.hpp cuts them on 256 CUs: R (row tiles of a raw wave, 0:
+# unpacked), parts of a split tile, passes over the rows.
+MX_CASES = [
+    ((256, 40, 65), (1, 1, 1)),       # one pair of blocks, less than a row tile of 32 and its wave
+    ((768, 300, 97), (1, 1, 1)),      # 6 blocks (rows not 16-byte aligned), a fourth token tile of one
+    ((2304, 8200, 31), (1, 5, 1)),    # 18 blocks, a ragged last panel
+    ((5120, 17408, 17), (1, 3, 1)),   # blocks in parts: raw, one row tile a wave
+    ((5120, 4100, 96), (1, 5, 1)),    # ragged panel, three token tiles
+    ((5120, 17408, 64), (2, 3, 1)),   # raw, two row tiles a wave
+    ((5120, 70000, 20), (2, 1, 1)),   # raw, several rounds of workgroups
+    ((5120, 1500, 3000), (0, 1, 1)),  # unpacked tiles, fewer than the CUs
+    ((5120, 8200, 1100), (0, 5, 1)),  # unpacked: a whole round, the rest in parts, ragged both ways
+    ((5120, 40000, 450), (2, 1, 1)),  # raw, whole tiles over eight rounds
+    ((5120, 40000, 640), (0, 8, 2)),  # unpacked in two passes over the rows, the second ragged
+    ((17408, 512, 2), (1, 23, 1)), ((17408, 700, 4), (1, 23, 1)),  # digits too long for LDS
+    ((5120, 2000, 20), (1, 20, 1)), ((5120, 4096, 1100), (0, 1, 1)),  # the zero-weight tests'
+]

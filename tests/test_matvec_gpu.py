@@ -285,24 +285,16 @@ def test_host_mirrors(bh, oracle, synth):
     assert _per_token_err(ym, oracle.pq2_matmul_n(table, ne0, n_rows, x)) <= TOL
 
 
-@pytest.mark.parametrize("ne0,n_rows,n_tok", [
-    (256, 40, 5),         # one pair of blocks, less than a row tile of 32 and its wave
-    (768, 300, 33),       # 6 blocks (rows not 16-byte aligned), a second token tile of one
-    (2304, 8200, 31),     # 18 blocks, a ragged last panel
-    (5120, 17408, 17),    # blocks in parts: raw, one row tile a wave
-    (5120, 4100, 96),     # ragged panel, three token tiles
-    (5120, 17408, 64),    # raw, two row tiles a wave
-    (5120, 70000, 20),    # raw, several rounds of workgroups
-    (5120, 1500, 3000),   # unpacked tiles, fewer than the CUs
-    (5120, 8200, 1100),   # unpacked: a whole round, the rest in parts, ragged both ways
-    (5120, 40000, 450),   # unpacked in two passes over the rows
-    (17408, 512, 2), (17408, 700, 4),  # digits too long for LDS
+@pytest.mark.parametrize("ne0,n_rows,n_tok", [c[0] for c in pq2data.MX_CASES] + [
+    # short rows that take the f16 form: its 16-token tiles, one and several
+    (256, 40, 5), (768, 300, 16), (768, 300, 33), (512, 8200, 64), (1280, 300, 9),
 ])
 def test_matmul_block_scaled(bh, synth, dev, ne0, n_rows, n_tok):
-    """The block-scaled forms at the edges of their tiles against 64-bit sums
-    of the same weights.  x has 24-bit digits and every f32 sum rounds once,
-    so the 2-norm error stays within sqrt(10) roundings of a block's sum and
-    sqrt(blocks) of a row's: (sqrt(10) + sqrt(nblk)) 2^-24."""
+    """The block-scaled forms (and the f16 one on short rows) at the edges of
+    their tiles against 64-bit sums of the same weights.  x has 24-bit digits
+    (22 bits in two f16) and every f32 sum rounds once, so the 2-norm error
+    stays within sqrt(10) roundings of a block's sum and sqrt(blocks) of a
+    row's: (sqrt(10) + sqrt(nblk)) 2^-24."""
     import torch
     _say("block-scaled", ne0, n_rows, n_tok)
     g = torch.Generator(device=dev)
@@ -327,13 +319,14 @@ def test_matmul_block_scaled(bh, synth, dev, ne0, n_rows, n_tok):
     assert rel <= (10 ** 0.5 + nblk ** 0.5) * 2.0 ** -24
 
 
-@pytest.mark.parametrize("n_tok", [20, 1100])
-def test_matmul_zero_weight_hides_outlier(bh, synth, dev, n_tok):
+@pytest.mark.parametrize("n_rows,n_tok", [(2000, 20), (4096, 1100)])
+def test_matmul_zero_weight_hides_outlier(bh, synth, dev, n_rows, n_tok):
     """A weight of zero takes nothing from its x, however large: a token with
     one value 1e20 times the rest, met by code 1 in every row, gives what it
-    gives with that value zero, bit for bit (on both block-scaled forms)."""
+    gives with that value zero, bit for bit, where the rest of its group of 32
+    columns is zero (on both block-scaled forms: raw, unpacked)."""
     import torch
-    ne0, n_rows = 5120, 2000
+    ne0 = 5120
     tab = torch.from_numpy(synth.pq2_table(synth.Rng(31), n_rows, ne0)).to(dev)
     col = 1234  # byte 2 + (1234 % 128) / 4 of block 9, code 2: bits 4-5
     byte = 34 * (col // 128) + 2 + (col % 128) // 4
@@ -345,3 +338,31 @@ def test_matmul_zero_weight_hides_outlier(bh, synth, dev, n_tok):
     x[:, col] = 1e20
     got = _h(bh.pq2_matmul_n(tab.view(-1), ne0, n_rows, x))
     assert np.array_equal(got, base)
+
+
+@pytest.mark.parametrize("n_rows,n_tok", [(2000, 20), (4096, 1100)])
+def test_matmul_outlier_beside_live_columns(bh, dev, n_rows, n_tok):
+    """One column of every group of 32 holds 1024 and meets a weight of zero.
+    The group's digits have a step of 2^-24 of the power of two above its
+    largest value, 2^(11 - 24): the other columns are rounded to it, an error of
+    2^-13 / sqrt(12) each, and no more than that reaches the outputs."""
+    import torch
+    ne0, nblk = 5120, 40
+    g = torch.Generator(device=dev)
+    g.manual_seed(n_rows + n_tok)
+    codes = torch.randint(0, 3, (n_rows, ne0), device=dev, generator=g, dtype=torch.uint8)
+    codes[:, 5::32] = 1
+    d = (torch.randn((n_rows, nblk), device=dev, generator=g) * 0.02).to(torch.float16)
+    c4 = codes.view(n_rows, nblk, 32, 4)
+    tab = torch.empty((n_rows, nblk, 34), device=dev, dtype=torch.uint8)
+    tab[..., :2] = d.view(torch.uint8).view(n_rows, nblk, 2)
+    tab[..., 2:] = c4[..., 0] | (c4[..., 1] << 2) | (c4[..., 2] << 4) | (c4[..., 3] << 6)
+    x = torch.randn((n_tok, ne0), device=dev, generator=g)
+    x[:, 5::32] = 1024.0
+    y = bh.pq2_matmul_n(tab.view(-1), ne0, n_rows, x)
+    w = ((codes.double() - 1).view(n_rows, nblk, 128) * d.double()[..., None]).view(n_rows, ne0)
+    ref = x.double() @ w.T
+    rel = float((y.double() - ref).norm() / ref.norm())
+    _say("outlier beside live columns", n_rows, n_tok, rel)
+    # 31 of 32 columns of unit variance; 10 % for the sample, and the sums' own rounding
+    assert rel <= 1.1 * 2.0 ** -13 / 12 ** 0.5 + 10 * 2.0 ** -24

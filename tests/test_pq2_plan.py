@@ -8,6 +8,8 @@ from pathlib import Path
 
 import pytest
 
+import pq2data
+
 SRC = Path(__file__).resolve().parent / "cpp" / "test_pq2_plan.cpp"
 
 
@@ -25,6 +27,15 @@ def test_scratch_grows_with_tokens(plan_exe):
     res = subprocess.run([str(plan_exe)], capture_output=True, text=True, timeout=120)
     print(res.stdout)
     assert res.returncode == 0 and "0 failures" in res.stdout, res.stdout
+
+
+@pytest.mark.parametrize("shape,plan", pq2data.MX_CASES)
+def test_products_reach_their_form(plan_exe, shape, plan):
+    """The shapes of the block-scaled products' GPU tests are cut as their list
+    says: a change of the plan's constants can't move one to another kernel
+    unnoticed."""
+    res = subprocess.run([str(plan_exe), *map(str, shape)], capture_output=True, text=True, check=True)
+    assert tuple(map(int, res.stdout.split())) == plan
 
 
 _CAPTURE_SCRIPT = r'''
