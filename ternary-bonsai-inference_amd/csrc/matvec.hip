@@ -11,7 +11,7 @@
 // well below 1e-5 of the output's largest magnitude).  Up to 4 tokens, and
 // few outputs or many row tiles of up to 16 tokens, run here on the integer
 // matrix cores; other batches in pq2_mx.hip on the block-scaled ones; the f16
-// form below takes up to 4 tokens on rows that cannot be staged.
+// form below takes up to 4 tokens, and short rows, that cannot be staged.
 //
 // Mapping onto v_mfma_f32_16x16x32_f16 (D = A * B + C, 16x16 output tile;
 // lane l holds A[l % 16][8 (l / 16) .. +7], B[8 (l / 16) .. +7][l % 16],
@@ -213,6 +213,11 @@ __device__ __forceinline__ BlockCodes block_codes(const PairData &d, int half) {
 
 template <int NT, bool ALDS>
 __global__ __launch_bounds__(kMmThreads) void pq2_mm_kernel(MmArgs a) {
+  // token tile blockIdx.y
+  a.afrag += static_cast<size_t>(blockIdx.y) * a.n_ksteps * 2 * 64;
+  a.binv += static_cast<size_t>(blockIdx.y) * a.nblk * 8;
+  a.y += static_cast<size_t>(blockIdx.y) * 16 * a.y_stride;
+  a.n_tok = a.n_tok - 16 * static_cast<int>(blockIdx.y) < 16 ? a.n_tok - 16 * static_cast<int>(blockIdx.y) : 16;
   // ALDS: the x side of the whole
   // product is staged in LDS once, fragments [kstep][piece][token][lane
   // group] followed by the block factors [block][lane group]
@@ -1178,9 +1183,10 @@ constexpr size_t kLdsABytes = 104 * 1024;  // LDS budget of a whole x side (with
 template <int NT, bool ALDS = false>
 int launch_mm(const MmArgs &a, hipStream_t st) {
   const unsigned gx = static_cast<unsigned>((a.n_rows + 64 * NT - 1) / (64 * NT));
+  const unsigned gy = static_cast<unsigned>((a.n_tok + 15) / 16);
   size_t lds = 0;
   if constexpr (ALDS) {
-    lds = static_cast<size_t>(a.n_ksteps) * 2 * a.n_tok * 4 * sizeof(uint4) +
+    lds = static_cast<size_t>(a.n_ksteps) * 2 * std::min(a.n_tok, 16) * 4 * sizeof(uint4) +
           static_cast<size_t>(a.nblk) * 8 * sizeof(float4);
     if (int e = check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(pq2_mm_kernel<NT, true>),
                                               hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1188,7 +1194,7 @@ int launch_mm(const MmArgs &a, hipStream_t st) {
                           "hipFuncSetAttribute"))
       return e;
   }
-  BH_LAUNCH((pq2_mm_kernel<NT, ALDS>), gx, kMmThreads, lds, st, a);
+  BH_LAUNCH((pq2_mm_kernel<NT, ALDS>), dim3(gx, gy), kMmThreads, lds, st, a);
   return ok();
 }
 
@@ -1353,27 +1359,41 @@ int pq2_mm(const uint8_t *w, size_t ne0, size_t n_rows, const float *x, size_t n
                            (nblk * kI8Tok * sizeof(float2) + 15) / 16 * 16;
     if (a_bytes <= kLdsABytes) return pq2_i8<false>(w, ne0, n_rows, x, n_tok, y, a_bytes, st);
   }
-  // more tokens, and rows so long that their digits don't fit LDS
-  // ([5120 x 17408], 4 tokens: 51 -> 27 us): the block-scaled matrix cores --
-  // except where the integer form is still faster: one pass over a matrix of
-  // many row tiles ([248320 x 5120], 16 tokens: 138 us against 146; [17408 x
-  // 5120]: 30 against 25), and short rows with few outputs, where its fewer
-  // launches count (2048 columns, 3000 x 300 outputs: 22 us against 25; 8000 x
-  // 300: 39 against 33).
-  if (n_tok > static_cast<size_t>(kI8Tok) || stageable) {
+  // Short rows that cannot be staged: the f16 form starts sooner than a pair of
+  // blocks passes the block-scaled kernel (us, f16 / block-scaled: 5120 x 768, 5
+  // tokens 9.0 / 12.7, 33 11.3 / 13.5; 17408 x 512, 33 11.3 / 12.2, 64 15.0 /
+  // 12.1; 5120 x 1280, 5 10.5 / 12.8, 10 12.5 / 12.9, 16 14.7 / 13.1; 65536 x
+  // 768, 16 17.4 / 13.9).
+  const bool f16 = !stageable && n_tok <= 64 && (nblk <= 6 || (nblk <= 14 && nblk * n_tok <= 96)) &&
+                   n_rows * n_tok * nblk <= (1u << 21);
+  // More tokens, and rows so long that their digits don't fit LDS (1 token on
+  // [1000 x 32768]: 88 -> 26 us, 4 on [5120 x 17408] 51 -> 26): the
+  // block-scaled matrix cores, whose error is the least (2-norm against 64
+  // bits on 40 blocks of normal x 1.2e-7, f16 1.7e-7, integer 3.0e-7) --
+  // except where the integer form is much faster.  It streams a matrix of many
+  // row tiles in one pass, but walks a row as one chain, so its line is in rows
+  // a block (us, integer / block-scaled: [248320 x 5120] 5 tokens 108 / 141, 16
+  // 146 / 151; [49152 x 5120] 8 33 / 43; [32768 x 8192] 8 40 / 40, 16 48 / 41;
+  // [32768 x 17408] 5 74 / 64; below 32768 rows it gains at most 5 % at the
+  // model's [17408 x 5120], 24 / 25 for 5 to 8 tokens).  And it takes short
+  // rows with few outputs, where its fewer launches count (2048 columns, 20480
+  // rows x 16 tokens 15 / 21; 3000 x 300 22 / 25; 8000 x 300 39 / 33).
+  if (!f16 && (n_tok > static_cast<size_t>(kI8Tok) || stageable)) {
     // items of the forms below and above, which index them in int
     if (n_tok * nblk * (stageable ? 8 : 16) > static_cast<size_t>(INT32_MAX) - kMmThreads)
       return fail(BH_ERR_SHAPE, "pq2_matmul_n: n_tok * ne0 too large for one call");
-    const bool i8 = (n_tok <= 16 && n_rows >= 32768) || (nblk <= 16 && n_rows * n_tok <= (1u << 20));
+    const bool i8 = (n_tok <= 16 && n_rows >= 32768 && n_rows >= 48 * nblk * std::max<size_t>(n_tok, 9)) ||
+                    (nblk <= 16 && n_rows * n_tok <= (1u << 20));
     if (stageable && n_tok > static_cast<size_t>(kI8Tok) && i8)
       return pq2_gemm_i8(w, ne0, n_rows, x, n_tok, y, st);
     return pq2_mx_gemm(w, ne0, n_rows, x, n_tok, y, st);
   }
-  // f16 hi / lo: up to 4 tokens on rows that cannot be staged
+  // f16 hi / lo
   const int n_ksteps = static_cast<int>(ne0 / 32);
-  const size_t frag_bytes = static_cast<size_t>(n_ksteps) * 2 * 64 * sizeof(uint4);
+  const size_t n_tiles = (n_tok + 15) / 16;
+  const size_t frag_bytes = n_tiles * n_ksteps * 2 * 64 * sizeof(uint4);
   const size_t binv_off = (frag_bytes + 255) / 256 * 256;
-  const size_t binv_bytes = nblk * 8 * sizeof(float4);
+  const size_t binv_bytes = n_tiles * nblk * 8 * sizeof(float4);
   char *scratch = static_cast<char *>(device_scratch(binv_off + binv_bytes, kScratchMatmul, st));
   if (scratch == nullptr) return BH_ERR_HIP;
   PrepArgs pa{x, reinterpret_cast<uint4 *>(scratch), reinterpret_cast<float *>(scratch + binv_off),
@@ -1389,7 +1409,7 @@ int pq2_mm(const uint8_t *w, size_t ne0, size_t n_rows, const float *x, size_t n
            static_cast<int>(n_rows)};
   // a wave takes 4 row tiles when that still leaves >= 2 blocks per CU
   const bool wide = n_rows >= static_cast<size_t>(256) * 2 * 256;
-  const bool a_in_lds = static_cast<size_t>(n_ksteps) * 2 * n_tok * 4 * sizeof(uint4) +
+  const bool a_in_lds = static_cast<size_t>(n_ksteps) * 2 * std::min<size_t>(n_tok, 16) * 4 * sizeof(uint4) +
                             nblk * 8 * sizeof(float4) <= kLdsABytes;
   if (a_in_lds)
     return wide ? launch_mm<4, true>(a, st) : launch_mm<1, true>(a, st);
