@@ -377,10 +377,12 @@ int bh_pq2_embed_gather_rms(const uint8_t *table, size_t ne0, size_t n_rows,
  * with the reference's scalar row dot to <= 1e-5 of the output's largest
  * magnitude (the summation order differs, as the reference's AVX2 path's
  * does).  Up to 4 tokens on rows of whole 1024-weight chunks (16-byte
- * aligned) the products keep x in LDS and use no scratch; otherwise they
- * use the library's per-device scratch (x fragments; for large batches also
- * up to 96 MB of unpacked weights, and partial sums): such calls must not
- * overlap on one device.
+ * aligned) the products keep x in LDS (up to 25600, 12288, 8192 and 6144
+ * columns for 1 to 4 tokens) and use no scratch; otherwise they use the
+ * library's per-device scratch (x fragments, up to 96 MB of partial sums; from
+ * 129 tokens also up to 96 MB of unpacked weights): such calls must not
+ * overlap on one device.  A call reserves what any smaller batch of the same
+ * matrix may need.
  * ------------------------------------------------------------------------- */
 
 /* kernels::pq2_matvec_range (src/kernels.rs:283-333):

@@ -1571,11 +1571,10 @@ __global__ __launch_bounds__(256) void attn_kv_split_kernel(const float *kc, con
 // the tiles in flight.  What bounds it now is instruction issue: a tile's
 // 64 products (f16) take 2048 cycles and its ~450 other vector instructions
 // about as many, of which half hides.
-// Measured, 24 / 4 heads: f16 cache, 333 queries at 4000: 102 us (16-row form
-// 122), at 12000: 245 (start of the tile loop to its end 2.3 us a tile
-// against 2.9); f32, 2048 queries from position 0: 230 us (270).  Relative
-// error against 64-bit arithmetic there 3.0e-7 (3.9e-7: the small cross
-// products have their own accumulator).
+// Measured, 24 / 4 heads, the kernel alone: f16 cache, 333 queries at 4000: 106
+// us (16-row form 122); f32, 2048 queries from position 0: 224 us (270).
+// Relative error against 64-bit arithmetic there 3.0e-7 (3.9e-7: the small
+// cross products have their own accumulator).
 constexpr int kWideThreads = 256;             // 4 waves, one per SIMD
 constexpr size_t kWideMinTiles = 8;           // position tiles per block from which this form is taken
 constexpr int kWideArr = 32 * kHd;            // halves of one operand array of a tile (16 KB)
@@ -1952,7 +1951,8 @@ __device__ __forceinline__ void mq_wide_body(const MqArgs &a) {
       if (s == 3) run_l += pair_sum(psum);
       if (s >= 1) unscale(s - 1);
       if (s >= 2) hide(s - 2);
-      // the buffers written here were last read before the previous barrier
+      // the buffers written here were last read before the barrier that this
+      // pass began behind
       constexpr int kFirst = 16 - kStageK - kStageV;
       if (s >= kFirst && s < kFirst + kStageK) stage_k(buf, s - kFirst);
       if (s >= kFirst + kStageK) stage_v(buf ^ 1, s - kFirst - kStageK);
@@ -2576,14 +2576,15 @@ extern "C" int bh_attention(const float *q, size_t n_q, size_t pos0, const void 
     const dim3 grid(static_cast<unsigned>(nb));
     // an f32 cache read by many row tiles per kv head (a prefill) is split
     // into f16 hi / lo once instead of in every block.  Blocks of eight and
-    // more position tiles take the 32-row form: its loop is faster (2.3 us a
-    // tile against 2.9 over an f16 cache) and its start and end cost 4 us
-    // more, q's fragments passing through LDS and the pipeline filling.
-    // Measured, 16-row / 32-row form, us a call with its q and k steps: 1 tile
-    // a block (16 queries at 1000, f16) 29.0 / 32.5, 3 (333 at 0) 48.4 / 51.5,
-    // 4 (22 at 4000) 38.7 / 40.5, 7 (64 at 4032) 47.7 / 47.6, 8 (512 at 0, f32)
-    // 78.3 / 77.1, 12 (200 at 2000, f32) 90.8 / 82.7, 15 (8 at 30000) 63.9 /
-    // 58.6, 35 (333 at 4000) 132.8 / 114.3, 64 (2048 at 0, f32) 304 / 264.
+    // more position tiles take the 32-row form: its loop is faster and its
+    // start and end cost 3 us more, q's fragments passing through LDS and the
+    // pipeline filling.  Measured, 24 / 4 heads, 16-row / 32-row form, us a
+    // call: 1 tile a block (16 queries at 1000, f16) 21.6 / 24.8, 3 (333 at 0)
+    // 35.5 / 38.3, 4 (22 at 4000) 31.9 / 34.4, 7 (64 at 4032) 40.4 / 42.6, 8
+    // (64 at 5312) 48.3 / 47.8, (512 at 0, f32) 63.4 / 64.3, 10 (333 at 947,
+    // f16) 55.7 / 55.1, (200 at 1720, f32) 71.1 / 69.9, 12 (200 at 2104, f32)
+    // 80.5 / 76.7, 14 (64 at 9344, f16) 59.7 / 58.4, 35 (333 at 4000) 119.8 /
+    // 105.8, 64 (2048 at 0, f32) 251 / 214, 149 (512 at 9000, f32) 583 / 461.
     const bool pre = !f16 && tiles_r >= kMqPreTiles;
     const bool wide = (f16 || pre) && per >= kWideMinTiles;
     if (pre && wide) {

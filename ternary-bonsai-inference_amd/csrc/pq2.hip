@@ -25,7 +25,7 @@
 // evaluates exactly without its additions.  Up to 16 rows per CU one launch:
 // a workgroup per row, one wave taking the row's runs by turns (a lane per
 // block; code 3 adds 4 d*d, see wave_row_ss) under the embedding stores, then
-// the norm row.  Its time is the launch, the row's first touch and about 15
+// the norm row.  Its time is the launch, the row's first touch and about 16
 // turns: T = 1 8.4 us, 256 11.5, 2048 17.2 (5.0 TB/s of 86.7 MB); a chain of
 // the 5120 additions, a lane per row, took 22.7, 27.8 and 29.5.  Longer
 // batches: two launches of flat writers (below), the sums walked a lane per
@@ -59,8 +59,8 @@ struct GatherArgs {
 };
 
 // Decodes float4 f of the packed row at `rowb` straight from global memory
-// (the scale halfword and one code byte; the row is 16-byte aligned and a
-// block starts on an even byte, so the halfword load is aligned).
+// (the scale halfword and one code byte; a block starts on an even byte, so
+// the halfword load is aligned).
 __device__ __forceinline__ float4 decode4_global(const uint8_t *rowb, int f) {
   const uint8_t *blk = rowb + (f >> 5) * kPq2Block;
   const uint32_t h = *reinterpret_cast<const uint16_t *>(blk);

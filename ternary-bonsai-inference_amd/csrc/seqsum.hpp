@@ -188,12 +188,12 @@ __host__ __device__ inline uint32_t repeat_add_step_f32(float &s, float x, uint3
 // them.  While the sum stays in its binade every run adds n m units whatever
 // the sum is, so a turn forms all m from the current binade, gives each lane
 // its start by an exclusive prefix sum, and applies all runs up to the first
-// that does not stay (it leaves the binade, or is a tie from an odd sum);
-// that run's own step then carries the sum on, and the next turn starts from
-// there.  A row of 40 blocks of model-like scales takes about 15 turns of some
-// 500 cycles instead of 55 dependent steps of some 900.  An increment is cut to
-// 2^25: past the end of the binade, where later starts no longer matter, and
-// 64 of them fit 32 bits.
+// that does not stay (it reaches the binade's end, or is a tie from an odd
+// sum); that run's own step then carries the sum on, and the next turn starts
+// from there.  A row of 40 blocks (scales |N(0, 0.02)|, three of five codes
+// not 1) takes 16 turns of some 500 cycles instead of 55 dependent steps of
+// some 900.  An increment is cut to 2^25: past the end of the binade, where
+// later starts no longer matter, and 64 of them fit 32 bits.
 __host__ __device__ inline uint32_t seq_units_added(uint32_t n, const SeqUnits &v) {
   const uint32_t inc = n * v.m;  // <= 256 * 2^24 only past the binade; n <= 128 fits 32 bits
   return inc < (1u << 25) ? inc : 1u << 25;
