@@ -48,8 +48,11 @@ inline int pow2ceil(size_t v) {
 // device must not overlap in time.  A buffer grows on demand (at least
 // twofold) and the buffer it replaces is kept until the process ends, so a
 // graph captured earlier keeps valid addresses.  Growth while `stream` is
-// capturing is refused (it would allocate inside the capture).  Returns
-// nullptr with the status recorded on failure.
+// capturing is refused (it would allocate inside the capture).  A caller may
+// ask for more than the call at hand needs, so that later ones find it: where
+// that cannot be had (a capture, no memory left) `least` bytes are enough (0:
+// all of them are needed).  Returns nullptr with the status recorded on
+// failure.
 constexpr int kScratchSoftmax = 0;  // split-row softmax partials
 constexpr int kScratchMatmul = 1;   // PQ2_0 product: x fragments and factors, unpacked rows, partial sums
 constexpr int kScratchAttention = 2;  // attention: chunk partials or probabilities
@@ -57,7 +60,7 @@ constexpr int kScratchGather = 3;     // gather + RMSNorm: the row scales
 constexpr int kScratchGdn = 4;        // gated delta-net chunks: prepared matrices
 constexpr int kScratchKvSplit = 5;    // attention: f32 cache split into f16 hi / lo
 constexpr int kScratchSlots = 6;
-void *device_scratch(size_t bytes, int slot, hipStream_t stream);
+void *device_scratch(size_t bytes, int slot, hipStream_t stream, size_t least = 0);
 // Current size of this device's buffer for `slot` (0 before the first use).
 size_t scratch_bytes(int slot);
 // Compute units of the current device (queried once per device; 256 if the

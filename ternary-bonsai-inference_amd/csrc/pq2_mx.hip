@@ -702,7 +702,7 @@ int pq2_mx_gemm(const uint8_t *w, size_t ne0, size_t n_rows, const float *x, siz
   const MxPlan plan = mx_plan(n_rows, n_tok, nblk, slots);
   const MxScratch m = mx_scratch_of(plan, n_rows, n_tok, nblk, slots);
   char *scratch = static_cast<char *>(
-      device_scratch(std::max(m.total(), mx_reserve_bytes(n_rows, n_tok, nblk)), kScratchMatmul, st));
+      device_scratch(mx_reserve_bytes(n_rows, n_tok, nblk), kScratchMatmul, st, m.total()));
   if (scratch == nullptr) return BH_ERR_HIP;
   if (plan.R == 1) return launch_raw<1>(w, ne0, n_rows, x, n_tok, y, plan.split, scratch, m, st);
   if (plan.R == 2) return launch_raw<2>(w, ne0, n_rows, x, n_tok, y, plan.split, scratch, m, st);

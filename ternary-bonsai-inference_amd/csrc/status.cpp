@@ -56,7 +56,8 @@ int check_launch(const char *what) {
   return check_hip(hipGetLastError(), what);
 }
 
-void *device_scratch(size_t bytes, int slot, hipStream_t stream) {
+void *device_scratch(size_t bytes, int slot, hipStream_t stream, size_t least) {
+  bytes = std::max(bytes, least);
   int dev = 0;
   if (check_hip(hipGetDevice(&dev), "hipGetDevice") != BH_OK) return nullptr;
   std::lock_guard<std::mutex> lock(g_scratch_mu);
@@ -71,6 +72,7 @@ void *device_scratch(size_t bytes, int slot, hipStream_t stream) {
   if (check_hip(hipStreamIsCapturing(stream, &cap), "hipStreamIsCapturing") != BH_OK)
     return nullptr;
   if (cap != hipStreamCaptureStatusNone) {
+    if (least != 0 && s.bytes >= least) return s.ptr;
     fail(BH_ERR_HIP, "scratch of " + std::to_string(bytes) + " bytes needed but " +
                          std::to_string(s.bytes) +
                          " reserved, and the stream is capturing: run this call once outside "
@@ -80,7 +82,14 @@ void *device_scratch(size_t bytes, int slot, hipStream_t stream) {
   size_t want = bytes < (1u << 20) ? (1u << 20) : bytes;
   if (s.bytes <= SIZE_MAX / 2 && want < 2 * s.bytes) want = 2 * s.bytes;
   void *p = nullptr;
-  if (check_hip(hipMalloc(&p, want), "scratch hipMalloc") != BH_OK) return nullptr;
+  hipError_t e = hipMalloc(&p, want);
+  if (e != hipSuccess && least != 0 && least < want) {
+    (void)hipGetLastError();  // the next launch check must not report this
+    if (s.bytes >= least) return s.ptr;
+    want = least;
+    e = hipMalloc(&p, want);
+  }
+  if (check_hip(e, "scratch hipMalloc") != BH_OK) return nullptr;
   // queued work and captured graphs may still use the old buffer: keep it
   if (s.ptr != nullptr) g_retired.push_back(Retired{s.ptr, s.bytes, dev});
   s.ptr = p;

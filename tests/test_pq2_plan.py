@@ -68,6 +68,18 @@ for t in (33, 17, 5):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, want), (t, rep)
+# a matrix never called before, which would reserve more than there is now and
+# needs less: the capture takes what is there
+n_rows = 20000
+tab = tab[:34].repeat(n_rows * ne0 // 128)
+x, y, s = torch.randn((100, ne0), device=dev), torch.empty((100, n_rows), device=dev), torch.cuda.Stream(device=dev)
+torch.cuda.synchronize()
+g = torch.cuda.CUDAGraph()
+with torch.cuda.graph(g, stream=s):
+    bh.pq2_matmul_n(tab, ne0, n_rows, x, out=y, stream=s)
+g.replay()
+torch.cuda.synchronize()
+assert torch.equal(y, bh.pq2_matmul_n(tab, ne0, n_rows, x))
 print("capture ok")
 '''
 
