@@ -1186,7 +1186,7 @@ int launch_mm(const MmArgs &a, hipStream_t st) {
   const unsigned gy = static_cast<unsigned>((a.n_tok + 15) / 16);
   size_t lds = 0;
   if constexpr (ALDS) {
-    lds = static_cast<size_t>(a.n_ksteps) * 2 * std::min(a.n_tok, 16) * 4 * sizeof(uint4) +
+    lds = static_cast<size_t>(a.n_ksteps) * 2 * a.n_tok * 4 * sizeof(uint4) +
           static_cast<size_t>(a.nblk) * 8 * sizeof(float4);
     if (int e = check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(pq2_mm_kernel<NT, true>),
                                               hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1360,12 +1360,17 @@ int pq2_mm(const uint8_t *w, size_t ne0, size_t n_rows, const float *x, size_t n
     if (a_bytes <= kLdsABytes) return pq2_i8<false>(w, ne0, n_rows, x, n_tok, y, a_bytes, st);
   }
   // Short rows that cannot be staged: the f16 form starts sooner than a pair of
-  // blocks passes the block-scaled kernel (us, f16 / block-scaled: 5120 x 768, 5
-  // tokens 9.0 / 12.7, 33 11.3 / 13.5; 17408 x 512, 33 11.3 / 12.2, 64 15.0 /
-  // 12.1; 5120 x 1280, 5 10.5 / 12.8, 10 12.5 / 12.9, 16 14.7 / 13.1; 65536 x
-  // 768, 16 17.4 / 13.9).
-  const bool f16 = !stageable && n_tok <= 64 && (nblk <= 6 || (nblk <= 14 && nblk * n_tok <= 96)) &&
-                   n_rows * n_tok * nblk <= (1u << 21);
+  // blocks passes the block-scaled kernel, as long as its rows, 16-token tiles
+  // (half of one up to 8 tokens, see a_in_lds) and blocks are few (us, f16 /
+  // block-scaled: 5120 x 768, 5 tokens 9.2 / 12.6, 33 9.8 / 13.4; 65536 x 768, 8
+  // 12.8 / 13.1, 10 14.9 / 13.2; 17408 x 768, 32 12.8 / 13.5, 33 15.1 / 14.0;
+  // 34816 x 512, 16 10.0 / 11.3, 17 13.1 / 11.3; 5120 x 1280, 8 11.1 / 12.8; 1024
+  // x 1792, 6 12.8 / 12.8).  One whole tile also wins where the block-scaled
+  // kernel cuts its panels in parts (5120 x 1280, 16 tokens 13.4 / 13.0; 12288 x
+  // 1280 13.5 / 16.1; 17408 x 1280 14.7 / 16.1; 34816 x 1280 18.0 / 16.3).
+  const bool f16 = !stageable && n_tok <= 64 &&
+                   n_rows * nblk * (n_tok <= 8 ? 1 : 2 * ((n_tok + 15) / 16)) <= 450000 &&
+                   (nblk <= 6 || (nblk <= 14 && nblk * n_tok <= 96) || (nblk <= 10 && n_tok <= 16 && n_rows > 8192));
   // More tokens, and rows so long that their digits don't fit LDS (1 token on
   // [1000 x 32768]: 88 -> 26 us, 4 on [5120 x 17408] 51 -> 26): the
   // block-scaled matrix cores, whose error is the least (2-norm against 64
@@ -1409,8 +1414,12 @@ int pq2_mm(const uint8_t *w, size_t ne0, size_t n_rows, const float *x, size_t n
            static_cast<int>(n_rows)};
   // a wave takes 4 row tiles when that still leaves >= 2 blocks per CU
   const bool wide = n_rows >= static_cast<size_t>(256) * 2 * 256;
-  const bool a_in_lds = static_cast<size_t>(n_ksteps) * 2 * std::min<size_t>(n_tok, 16) * 4 * sizeof(uint4) +
-                            nblk * 8 * sizeof(float4) <= kLdsABytes;
+  // x in LDS: each workgroup copies all of it first, which costs more than its
+  // rows' reads from L2 from some 10 tokens on (us, LDS / L2: 5120 x 768, 8 tokens
+  // 9.2 / 10.0, 10 9.6 / 9.8, 16 10.8 / 9.8, 64 12.2 / 11.0; 12288 x 1280, 8 11.1 /
+  // 13.4, 16 14.6 / 13.5)
+  const bool a_in_lds = n_tok <= 10 && static_cast<size_t>(n_ksteps) * 2 * n_tok * 4 * sizeof(uint4) +
+                                               nblk * 8 * sizeof(float4) <= kLdsABytes;
   if (a_in_lds)
     return wide ? launch_mm<4, true>(a, st) : launch_mm<1, true>(a, st);
   return wide ? launch_mm<4>(a, st) : launch_mm<1>(a, st);

@@ -287,7 +287,9 @@ def test_host_mirrors(bh, oracle, synth):
 
 @pytest.mark.parametrize("ne0,n_rows,n_tok", [c[0] for c in pq2data.MX_CASES] + [
     # short rows that take the f16 form: its 16-token tiles, one and several
+    # up to 10 tokens with x in LDS, more from L2
     (256, 40, 5), (768, 300, 16), (768, 300, 33), (512, 8200, 64), (1280, 300, 9),
+    (768, 8300, 10), (768, 8300, 11), (1280, 8200, 16),
 ])
 def test_matmul_block_scaled(bh, synth, dev, ne0, n_rows, n_tok):
     """The block-scaled forms (and the f16 one on short rows) at the edges of
