@@ -1378,17 +1378,24 @@ int pq2_mm(const uint8_t *w, size_t ne0, size_t n_rows, const float *x, size_t n
   // except where the integer form is much faster.  It streams a matrix of many
   // row tiles in one pass, but walks a row as one chain, so its line is in rows
   // a block (us, integer / block-scaled: [248320 x 5120] 5 tokens 108 / 141, 16
-  // 146 / 151; [49152 x 5120] 8 33 / 43; [32768 x 8192] 8 40 / 40, 16 48 / 41;
-  // [32768 x 17408] 5 74 / 64; below 32768 rows it gains at most 5 % at the
-  // model's [17408 x 5120], 24 / 25 for 5 to 8 tokens).  And it takes short
-  // rows with few outputs, where its fewer launches count (2048 columns, 20480
-  // rows x 16 tokens 15 / 21; 3000 x 300 22 / 25; 8000 x 300 39 / 33).
+  // 146 / 151; [49152 x 5120] 8 33 / 43; [24576 x 4096] 8 20 / 26, 16 25 / 26;
+  // [24576 x 5120] 8 24 / 27, 12 27 / 27; [32768 x 8192] 8 40 / 40, 16 48 / 41;
+  // [32768 x 17408] 5 74 / 64; on fewer rows it gains at most 5 % at the model's
+  // [17408 x 5120], 24 / 25 for 5 to 8 tokens).  And it takes short rows with
+  // few outputs, where its fewer launches count (2048 columns, 20480 rows x 16
+  // tokens 15 / 21; 3000 x 300 22 / 25; 8000 x 300 39 / 33; 1024 columns, 34816 x
+  // 33 16 / 20, 17408 x 72 15.0 / 16.4, 49152 x 32 15.2 / 15.9, 65536 x 17 16.4 /
+  // 15.5).
+  // (Between 17 and 100 tokens the block-scaled kernel's padding to 32 tokens and
+  // its whole rounds leave single shapes of 8 to 40 blocks where the integer form
+  // would be up to a quarter faster, [34816 x 2048] at 97 48 / 60; none on the
+  // model's rows.)
   if (!f16 && (n_tok > static_cast<size_t>(kI8Tok) || stageable)) {
     // items of the forms below and above, which index them in int
     if (n_tok * nblk * (stageable ? 8 : 16) > static_cast<size_t>(INT32_MAX) - kMmThreads)
       return fail(BH_ERR_SHAPE, "pq2_matmul_n: n_tok * ne0 too large for one call");
-    const bool i8 = (n_tok <= 16 && n_rows >= 32768 && n_rows >= 48 * nblk * std::max<size_t>(n_tok, 9)) ||
-                    (nblk <= 16 && n_rows * n_tok <= (1u << 20));
+    const bool i8 = (n_tok <= 16 && n_rows >= 24576 && n_rows >= 48 * nblk * std::max<size_t>(n_tok, 9)) ||
+                    (nblk <= 16 && n_rows * n_tok <= (nblk <= 8 && n_rows < 65536 ? 3u << 19 : 1u << 20));
     if (stageable && n_tok > static_cast<size_t>(kI8Tok) && i8)
       return pq2_gemm_i8(w, ne0, n_rows, x, n_tok, y, st);
     return pq2_mx_gemm(w, ne0, n_rows, x, n_tok, y, st);

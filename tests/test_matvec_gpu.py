@@ -108,6 +108,8 @@ def test_matmul_token_counts(bh, oracle, synth, dev, n_tok):
     (2048, 129, 260),     # 65 token groups: a second launch row of sets, one live group
     (17408, 48, 9),       # ffn_down's width, 136 blocks, three groups
     (1024, 5, 5),         # fewer rows than one tile, a group and one token
+    (2560, 24601, 7),     # many row tiles from 24576 rows on
+    (1024, 12301, 101),   # short rows past 2^20 outputs
 ])
 def test_matmul_prefill_shapes(bh, oracle, synth, dev, ne0, n_rows, n_tok):
     """The integer product for more than 4 tokens: x fragments prepared once
