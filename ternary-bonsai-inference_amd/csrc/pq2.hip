@@ -228,7 +228,8 @@ __device__ __forceinline__ float wave_row_ss(const uint8_t *row, int ne0, int nb
   return s;
 }
 
-__global__ __launch_bounds__(kRowThreads) void pq2_gather_row_kernel(GatherArgs a) {
+template <int T>
+__global__ __launch_bounds__(T) void pq2_gather_row_kernel(GatherArgs a) {
   __shared__ float row_scale;
   __shared__ __attribute__((aligned(16))) HandLds hand;
   const size_t t = blockIdx.x;
@@ -238,7 +239,7 @@ __global__ __launch_bounds__(kRowThreads) void pq2_gather_row_kernel(GatherArgs 
   float4 *on = reinterpret_cast<float4 *>(a.out_norm) + t * n4;
   if (id >= a.n_rows) {
     if (threadIdx.x == 0 && a.bad_id != nullptr) *a.bad_id = id;
-    for (int f = threadIdx.x; f < n4; f += kRowThreads) {
+    for (int f = threadIdx.x; f < n4; f += T) {
       store_stream(oe + f, make_float4(0.f, 0.f, 0.f, 0.f));
       store_stream(on + f, make_float4(0.f, 0.f, 0.f, 0.f));
     }
@@ -252,11 +253,11 @@ __global__ __launch_bounds__(kRowThreads) void pq2_gather_row_kernel(GatherArgs 
     if (threadIdx.x == 0) row_scale = 1.0f / sqrtf(ss / static_cast<float>(a.ne0) + a.eps);
     __builtin_amdgcn_s_setprio(0);
   } else {
-    for (int f = threadIdx.x - 64; f < n4; f += kRowThreads - 64) store_stream(oe + f, decode4_global(row, f));
+    for (int f = threadIdx.x - 64; f < n4; f += T - 64) store_stream(oe + f, decode4_global(row, f));
   }
   __syncthreads();
   const float rs = row_scale;
-  for (int f = threadIdx.x; f < n4; f += kRowThreads) {
+  for (int f = threadIdx.x; f < n4; f += T) {
     const float4 wv = reinterpret_cast<const float4 *>(a.w)[f];
     const float4 v = decode4_global(row, f);
     // src/kernels.rs:71-73
@@ -592,7 +593,17 @@ int gather_impl(const uint8_t *table, size_t ne0, size_t n_rows, const uint32_t 
     return ok();
   }
   if (rows_ok && norm && row_bytes % 4 == 0) {  // a block's codes are whole aligned words
-    BH_LAUNCH(pq2_gather_row_kernel, grid, kRowThreads, 0, st, ga);
+    // More rows than the CUs hold workgroups of 256 lanes (8 each): short ones
+    // take 128, so that all of them are under way at once.  2048 columns, us at
+    // 2560 / 3072 / 4095 rows of three codes: 17.1 / 18.4 / 21.7 with 256 lanes,
+    // 14.6 / 14.8 / 18.8 with 128; at 2048 rows 13.0 / 13.4, and 3072 columns at
+    // 4095 rows 22.8 / 25.3, so both lines stay there.  (A wave a row and a chain
+    // of all additions, a lane a row, were 22.3 and 17.0; that chain is the
+    // faster one on 1024 columns too, 11.4 for 15.1 at 4095 rows.)
+    if (n_ids > 8 * cus && ne0 <= 2048)
+      BH_LAUNCH((pq2_gather_row_kernel<128>), grid, 128, 0, st, ga);
+    else
+      BH_LAUNCH((pq2_gather_row_kernel<kRowThreads>), grid, kRowThreads, 0, st, ga);
   } else {
     if (norm) {
       BH_LAUNCH((pq2_gather_loop_kernel<true>), grid, kBlock, 0, st, table, row_bytes,

@@ -29,7 +29,7 @@ def test_row_by_turns_matches_sequential_loop(tmp_path, rcp_ulp):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("ne0", [256, 1272, 5120, 64 * 128, 70 * 128])
-@pytest.mark.parametrize("n_ids", [1, 5, 700])
+@pytest.mark.parametrize("n_ids", [1, 5, 700, 2500])  # 2500: more than 8 a CU, 128 lanes for short rows
 def test_gather_rms_row_kernel(bh, oracle, dev, ne0, n_ids):
     """One workgroup per row: rows of 2 blocks, a partial last block on rows
     that start on 4 bytes only, exactly one window of 64 blocks and a second
