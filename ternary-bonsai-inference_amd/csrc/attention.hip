@@ -1576,7 +1576,7 @@ __global__ __launch_bounds__(256) void attn_kv_split_kernel(const float *kc, con
 // Relative error against 64-bit arithmetic there 3.0e-7 (3.9e-7: the small
 // cross products have their own accumulator).
 constexpr int kWideThreads = 256;             // 4 waves, one per SIMD
-constexpr size_t kWideMinTiles = 8;           // position tiles per block from which this form is taken
+constexpr size_t kWideMinTiles = 10;          // position tiles per block from which this form is taken
 constexpr int kWideArr = 32 * kHd;            // halves of one operand array of a tile (16 KB)
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
@@ -2575,16 +2575,15 @@ extern "C" int bh_attention(const float *q, size_t n_q, size_t pos0, const void 
     if (nb > 0x7fffffffu) return fail(BH_ERR_SHAPE, "attention: too many blocks");
     const dim3 grid(static_cast<unsigned>(nb));
     // an f32 cache read by many row tiles per kv head (a prefill) is split
-    // into f16 hi / lo once instead of in every block.  Blocks of eight and
-    // more position tiles take the 32-row form: its loop is faster and its
-    // start and end cost 3 us more, q's fragments passing through LDS and the
-    // pipeline filling.  Measured, 24 / 4 heads, 16-row / 32-row form, us a
-    // call: 1 tile a block (16 queries at 1000, f16) 21.6 / 24.8, 3 (333 at 0)
-    // 35.5 / 38.3, 4 (22 at 4000) 31.9 / 34.4, 7 (64 at 4032) 40.4 / 42.6, 8
-    // (64 at 5312) 48.3 / 47.8, (512 at 0, f32) 63.4 / 64.3, 10 (333 at 947,
-    // f16) 55.7 / 55.1, (200 at 1720, f32) 71.1 / 69.9, 12 (200 at 2104, f32)
-    // 80.5 / 76.7, 14 (64 at 9344, f16) 59.7 / 58.4, 35 (333 at 4000) 119.8 /
-    // 105.8, 64 (2048 at 0, f32) 251 / 214, 149 (512 at 9000, f32) 583 / 461.
+    // into f16 hi / lo once instead of in every block.  Blocks of ten and more
+    // position tiles take the 32-row form: its loop is faster and its start and
+    // end cost 3 us more, q's fragments passing through LDS and the pipeline
+    // filling.  Measured, 32-row over 16-row time in calls of 2 to 2000 queries
+    // at 0 to 30000, five shapes of 8 to 32 heads: 8 tiles a block 1.00 - 1.07
+    // (median 1.03; 64 queries at 8000, 8 / 8 heads 40.1 / 37.0 us), 9 1.00 -
+    // 1.03, 10 0.99 - 1.02, 12 0.96 - 1.01, 15 0.95 - 1.00, 20 0.94, 32 0.82 -
+    // 0.93, 40 and more 0.73 - 0.93 (24 / 4 heads: 333 at 4000, f16 105.8 /
+    // 119.8; 2048 at 0, f32 214 / 251; 512 at 9000, f32 461 / 583).
     const bool pre = !f16 && tiles_r >= kMqPreTiles;
     const bool wide = (f16 || pre) && per >= kWideMinTiles;
     if (pre && wide) {

@@ -259,9 +259,9 @@ def test_attention_presplit_tile_scales(bh, oracle, synth, dev):
     (172, 90, False, 64.0),  # each tile's scores far above the last one's
     (171, 30, False, 0.0),   # seven tiles a block: the 16-row form
 ])
-def test_attention_wide_rows(bh, oracle, synth, dev, n_q, pos0, f16, span):
-    """The 32-row matrix-core form (blocks of eight and more position tiles
-    over f16 caches and f32 caches split beforehand; 32 kv heads, so that few
+def test_attention_wide_rows(bh, oracle, synth, dev, n_q, pos0, f16, span, n_kv=32):
+    """The matrix-core forms (16-row ones on blocks of up to nine position
+    tiles, the 32-row one from ten on, over f16 caches and f32 caches split beforehand; 32 kv heads, so that few
     positions make such blocks) at the edges of its row and position tiles, and with keys whose scores
     climb by `span` nats from the first position to the last, so that the
     running reference and the accumulators move many times.  A score of s
@@ -269,7 +269,7 @@ def test_attention_wide_rows(bh, oracle, synth, dev, n_q, pos0, f16, span):
     probability, times the few roundings of its sum: centred, |s| <= 42, and
     the oracle is within 6e-6 of 64-bit arithmetic on these inputs (at the
     uncentred |s| of 390 it is 1e-4 away, past TOL by itself)."""
-    n_head, n_kv, hd = 192, 32, 256
+    n_head, hd = 6 * n_kv, 256
     _say("attention wide rows", n_q, pos0, "f16" if f16 else "f32", span)
     q, kc, vc = _case(synth, n_q, pos0, n_head, n_kv, hd, 1500 + n_q + pos0, qscale=1.0)
     if span:
@@ -290,7 +290,24 @@ def test_attention_wide_rows(bh, oracle, synth, dev, n_q, pos0, f16, span):
     assert err <= TOL
 
 
-@pytest.mark.parametrize("n_q,pos0,f16", [(22, 1100, True), (256, 0, False)])
+@pytest.mark.parametrize("n_q,pos0,f16,span,n_kv", [
+    (8, 2873, True, 0.0, 25),     # ten tiles a block, 48 rows (two waves of four); the last chunk is one position
+    (8, 2552, True, 0.0, 32),     # whole tiles only
+    (11, 2300, True, 0.0, 32),    # 66 rows: a wave of two rows; a last chunk of three tiles
+    (22, 1200, True, 0.0, 32),    # 132 rows: a second row tile of four rows; a 6-position last tile
+    (64, 1100, True, 32.0, 32),   # scores that rise with the position: the reference moves many times
+    (8, 2240, True, 0.0, 32),     # nine tiles a block: the 16-row form
+    (320, 0, False, 0.0, 32),     # a pre-split f32 cache, causal from position 0, one chunk
+    (171, 118, False, 32.0, 32),  # its last tile holds one position
+    (172, 154, False, 64.0, 32),  # each tile's scores far above the last one's
+    (171, 100, False, 0.0, 32),   # nine tiles a block: the 16-row form
+])
+def test_attention_wide_rows_ten_tiles(bh, oracle, synth, dev, n_q, pos0, f16, span, n_kv):
+    """The same edges on blocks of ten tiles and more, and of nine."""
+    test_attention_wide_rows(bh, oracle, synth, dev, n_q, pos0, f16, span, n_kv)
+
+
+@pytest.mark.parametrize("n_q,pos0,f16", [(22, 1200, True), (320, 0, False)])
 def test_attention_wide_rows_first_tile(bh, oracle, synth, dev, n_q, pos0, f16):
     """The 32-row form's first staged tile is read by every wave before the
     third takes its place: most of each row's weight is on the first tile of
@@ -325,12 +342,12 @@ def test_attention_wide_rows_sink_and_flat_tail(bh, dev, f16):
     zero value, and a flat tail behind it, whose probabilities of 2^-15 to
     2^-19 are all rounded the same way.  In units of 2^-14 a probability p
     splits into two f16 with an error of 2^-25 at most: 2^-39 / p, 2^-20 of it
-    at the smallest p here.  The eight tiles are 32 products, each of which
+    at the smallest p here.  The ten tiles are 40 products, each of which
     rounds an f32 sum once: 2^-24 each at most; exponential, row sum and
     division are 8 more.  Scores are exact (multiples of 2^-8), the reference
     is in 64 bits."""
     import torch
-    n, n_head, n_kv, hd = 256, 192, 32, 256
+    n, n_head, n_kv, hd = 320, 192, 32, 256
     rng = np.random.default_rng(5)
     delta = np.round(rng.uniform(15, 19, (n, n_head)) * np.log(2.0) * 256) / 256
     q = np.zeros((n, n_head, hd), np.float32)
@@ -348,7 +365,7 @@ def test_attention_wide_rows_sink_and_flat_tail(bh, dev, f16):
     ref = (tail / (1.0 + tail))[..., None] * np.repeat(vals.reshape(n_kv, hd), n_head // n_kv, axis=0)
     rel = np.abs(got[1:] / ref[1:] - 1.0).max()
     _say("sink and tail", "f16" if f16 else "f32", rel)
-    assert rel <= 2.0 ** -20 + 40 * 2.0 ** -24
+    assert rel <= 2.0 ** -20 + 48 * 2.0 ** -24
 
 
 _SPLIT_CAPTURE_SCRIPT = r'''
