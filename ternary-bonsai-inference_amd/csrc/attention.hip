@@ -1978,10 +1978,11 @@ __device__ __forceinline__ void mq_wide_body(const MqArgs &a) {
 #pragma unroll
       for (int i4 = 0; i4 < 4; ++i4) {
         f32x4 v = {o[dt][4 * i4], o[dt][4 * i4 + 1], o[dt][4 * i4 + 2], o[dt][4 * i4 + 3]};
-        v = v * u;
-        // the merge of one chunk: weight e^0 = 1, so (acc * 1) / (l * 1)
-        // (the merge's 0 + acc turns an exact -0 into +0; nothing else differs)
-        if (fin) v = v / run_l;
+        // one chunk: the merge's (acc * 1) / (l * 1), weight e^0 = 1 (its 0 + acc
+        // turns an exact -0 into +0; nothing else differs), divided before the
+        // power of two: l counts probabilities of up to 3.9 and acc in V's own
+        // units could pass the largest f32 where the result does not
+        v = fin ? (v / run_l) * u : v * u;
         dst[8 * dt + 2 * i4 + h] = v;
       }
   }

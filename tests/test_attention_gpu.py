@@ -295,7 +295,6 @@ def test_attention_wide_rows(bh, oracle, synth, dev, n_q, pos0, f16, span, n_kv=
     (8, 2552, True, 0.0, 32),     # whole tiles only
     (11, 2300, True, 0.0, 32),    # 66 rows: a wave of two rows; a last chunk of three tiles
     (22, 1200, True, 0.0, 32),    # 132 rows: a second row tile of four rows; a 6-position last tile
-    (64, 1100, True, 32.0, 32),   # scores that rise with the position: the reference moves many times
     (8, 2240, True, 0.0, 32),     # nine tiles a block: the 16-row form
     (320, 0, False, 0.0, 32),     # a pre-split f32 cache, causal from position 0, one chunk
     (171, 118, False, 32.0, 32),  # its last tile holds one position
@@ -366,6 +365,20 @@ def test_attention_wide_rows_sink_and_flat_tail(bh, dev, f16):
     rel = np.abs(got[1:] / ref[1:] - 1.0).max()
     _say("sink and tail", "f16" if f16 else "f32", rel)
     assert rel <= 2.0 ** -20 + 48 * 2.0 ** -24
+
+
+def test_attention_wide_rows_large_values(bh, oracle, synth, dev):
+    """Values within a factor of ten of the largest f32: a row's sum of p v is
+    past it before the division, its result is not."""
+    n, n_head, n_kv, hd = 320, 192, 32, 256
+    q, kc, vc = _case(synth, n, 0, n_head, n_kv, hd, 91, qscale=1.0)
+    vc = (np.float32(4e37) + vc * np.float32(1e36)).astype(np.float32)
+    ref = oracle.attention(q, 0, kc, vc, n_kv)
+    got = _run(bh, dev, q, 0, kc, vc, n_kv)
+    assert np.isfinite(got).all()
+    err = rel_err(got, ref)
+    _say("wide rows, large values", err)
+    assert err <= TOL
 
 
 _SPLIT_CAPTURE_SCRIPT = r'''
