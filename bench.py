@@ -430,7 +430,7 @@ def _time_cpu(run, n_units: int, seconds: float):
         n_thr = len(os.sched_getaffinity(0))
     except AttributeError:
         n_thr = os.cpu_count() or 1
-    n_thr = max(1, min(n_thr, 16, n_units))  # the GPU box's CPU share is 16 cores
+    n_thr = max(1, min(n_thr, 16, n_units))  # a share of 16 cores
     cuts = [n_units * i // n_thr for i in range(n_thr + 1)]
     reps_mt, t1 = 0, time.perf_counter()
     with concurrent.futures.ThreadPoolExecutor(n_thr) as pool:

@@ -548,7 +548,7 @@ int gather_impl(const uint8_t *table, size_t ne0, size_t n_rows, const uint32_t 
   const unsigned grid = static_cast<unsigned>(n_ids);
   const uint32_t nr = static_cast<uint32_t>(n_rows);
   // writers: one float4 per lane (16-byte stores, halfword table loads); the
-  // fused kernel stages rows with 16-byte loads
+  // two-launch form stages rows with 16-byte loads
   const bool rows_ok = (ne0 % 4 == 0) && n_ids * (ne0 / 4) < 0xfffff000u && aligned16(table) &&
                        aligned16(out) && (!norm || (aligned16(out_norm) && aligned16(w)));
   const unsigned wgrid = static_cast<unsigned>((n_ids * (ne0 / 4) + 255) / 256);

@@ -1,4 +1,4 @@
-"""Pins the CPU oracle (oracle/oracle.c) before it is trusted as the checker.
+"""Pins the CPU oracle (oracle/oracle.c) before the kernels are compared with it.
 
 Every check comes from outside the oracle's own formulas:
   * the reference's unit tests, restated with their literal inputs/answers
